@@ -88,7 +88,19 @@ def _k(rng, lo, hi):
     return 256 * max(1, round(_log(rng, lo, hi) / 256))
 
 
+# no drawn case is larger than the largest listed one of its kind of arithmetic
+MOST_BYTES, MOST_FLOPS = 4.4e8, {"exact": 4.7e9, "int8": 1.1e10, "mfma": 2.3e10}
+
+
 def draw(rng):
+    while True:
+        c = _draw(rng)
+        w = work(c)
+        if w["bytes"] <= MOST_BYTES and w["flops"] <= MOST_FLOPS[c.get("mode", "exact")]:
+            return c
+
+
+def _draw(rng):
     kind = rng.choice(["host", "layer", "gemv", "gemv", "multi", "multi", "multi", "moe", "moe"])
     if kind == "host":
         t = rng.choice(list(TYPES))
