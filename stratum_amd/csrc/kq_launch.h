@@ -71,6 +71,13 @@ int kqk_launch_mx(int type, const int* plan, long lds, int grid, const void* w, 
                   const void* gdev, const int* ngdev, const float* X, long x_stride, float* Y,
                   long y_stride, int N, int K, hipStream_t st);
 int kqk_mx_set_max_lds(int bytes);
+/* exact MULTISEQ (kq_mv.hip): plan[] (kqk_mv_plan returns the LDS bytes, or
+ * -1: not taken), and the launch (x_j = X + j x_stride, y_j = Y + j y_stride) */
+#define KQK_MV_PLAN 5
+long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan);
+int kqk_mv_set_max_lds(int bytes);
+int kqk_launch_mv(int type, const int* plan, long lds, const void* w, const float* X, long x_stride,
+                  float* Y, long y_stride, int M, int N, int K, hipStream_t st);
 /* MoE: top-k per token; the expert groups (MxGroup records) of a selection */
 int kqk_launch_moe_topk(const float* probs, int B, int E, int k, int* sel, float* selw,
                         hipStream_t st);

@@ -220,7 +220,7 @@ static int kq_ready(void) {
     g_kq.n_cu = ncu > 0 ? ncu : 1;
     g_kq.lds_max = lds > 0 ? lds : 65536;
     if (kqk_set_max_lds(g_kq.lds_max) != 0 || kqk_mx_set_max_lds(g_kq.lds_max) != 0 ||
-        kqk_dense_set_max_lds(g_kq.lds_max) != 0)
+        kqk_dense_set_max_lds(g_kq.lds_max) != 0 || kqk_mv_set_max_lds(g_kq.lds_max) != 0)
         return kq_fail("cannot raise the LDS limit");
     /* the static scratch of the no-allocation entry point: its address on
      * this device, looked up once now (other devices at their first call) */
@@ -610,6 +610,34 @@ static long mx_plan(int type, int N, int K, int mmax, int ngmax, int grid, const
     return lds;
 }
 
+/* The exact MULTISEQ kernel's plans, kept like the multi-x ones. */
+typedef struct {
+    int used, type, N, K, B, n_cu, lds_max, plan[KQK_MV_PLAN];
+    long lds;
+} mv_plan_entry;
+static mv_plan_entry g_mv_plans[MX_PLAN_CACHE];
+static int g_mv_next;
+
+static long mv_plan(int type, int N, int K, int B, int* plan) {
+    for (int i = 0; i < MX_PLAN_CACHE; i++) {
+        const mv_plan_entry* c = &g_mv_plans[i];
+        if (c->used && c->type == type && c->N == N && c->K == K && c->B == B &&
+            c->n_cu == g_kq.n_cu && c->lds_max == g_kq.lds_max) {
+            memcpy(plan, c->plan, sizeof c->plan);
+            return c->lds;
+        }
+    }
+    memset(plan, 0, KQK_MV_PLAN * sizeof *plan);
+    const long lds = kqk_mv_plan(type, N, K, B, g_kq.n_cu, g_kq.lds_max, plan);
+    mv_plan_entry* c = &g_mv_plans[g_mv_next];
+    g_mv_next = (g_mv_next + 1) % MX_PLAN_CACHE;
+    c->used = 1; c->type = type; c->N = N; c->K = K; c->B = B;
+    c->n_cu = g_kq.n_cu; c->lds_max = g_kq.lds_max;
+    c->lds = lds;
+    memcpy(c->plan, plan, sizeof c->plan);
+    return lds;
+}
+
 static int mfma_reserve(kq_scr* sc, size_t need);
 
 /* The int8 MULTISEQ of st_linear_multix under use_sdot (Q4_K / Q6_K, B >= 2,
@@ -628,8 +656,9 @@ static int mi8_multix(int type, const void* w, const float* xs, float* ys, int B
     return 0;
 }
 
-/* B streams with one pass over the weights per group of up to 64 streams
- * (the multi-x kernel); each stream's y equals its single-stream result bit
+/* B streams with one pass over the weights: exact block types in kq_mv.hip
+ * (rows whose x sums leave no room for its tiles, and the int8 mode of Q5_K,
+ * Q3_K and Q8_0, in the multi-x kernel); each stream's y equals its single-stream result bit
  * for bit, except in the int8 mode of Q4_K / Q6_K (mi8_multix). */
 int kq_gemv_multix_dev(int type, const void* w, const float* xs, float* ys,
                        int B, int N, int K, kq_stream stream) {
@@ -645,6 +674,15 @@ int kq_gemv_multix_dev(int type, const void* w, const float* xs, float* ys,
             if (kq_gemv_dev(type, w, xs + (size_t)s * K, NULL, ys + (size_t)s * N, N, K, stream))
                 return -1;
         return 0;
+    }
+    if (!(type & KQ_INT8_ACT)) {
+        int plan[KQK_MV_PLAN];
+        const long lds = mv_plan(type, N, K, B, plan);
+        if (lds > 0) {
+            const int e = kqk_launch_mv(type, plan, lds, w, xs, K, ys, N, B, N, K, pick(stream));
+            if (e) return kq_fail("multix launch: %s", hipGetErrorString((hipError_t)e));
+            return 0;
+        }
     }
     const int grid = plan_grid();
     for (int s0 = 0; s0 < B; ) {
