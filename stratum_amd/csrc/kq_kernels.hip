@@ -3881,6 +3881,53 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
+// A few rows (a MoE router: at most DENSE_FEW_WAVES waves per CU): the launch
+// is one memory round trip, so a wave asks for BLK weight and x pieces of its
+// row at once, straight to registers, with no staging and no barrier.  The
+// sum runs in kq_dense_kernel's order.  128 x 2048 F32 (1 MB), B = 1, in a
+// MoE step: 7.2 us with x staged in LDS and the loads one at a time -> 3.9.
+constexpr int DENSE_FEW_WAVES = 8;
+template <int TYPE>
+__global__ __launch_bounds__(256) void kq_dense_few_kernel(DenseArg a) {
+    constexpr int E = TYPE == T_F32 ? 4 : 8, BLK = TYPE == T_F32 ? 8 : 4;
+    const int lane = threadIdx.x & 63, K = a.K, s = blockIdx.y;
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= a.N) return;
+    const wptr row = to_global(a.w) + (size_t)r * a.row_bytes;
+    const wptr xg = to_global(reinterpret_cast<const uint8_t*>(a.x + (size_t)s * K));
+    const float addv = a.add ? a.add[r] : 0.0f;
+    double acc = 0.0;
+    for (int m0 = 0; m0 < K; m0 += 64 * E * BLK) {
+        uint4 wv[BLK];
+        f32x4 xv[BLK][E / 4];
+#pragma unroll
+        for (int j = 0; j < BLK; j++) {                 // clamped: branch-free
+            const int e = min(m0 + E * (lane + 64 * j), K - E);
+            wv[j] = ld16(row + (size_t)e * (TYPE == T_F32 ? 4 : 2));
+#pragma unroll
+            for (int q = 0; q < E / 4; q++) xv[j][q] = wload<f32x4>(xg + 4 * (size_t)(e + 4 * q));
+        }
+#pragma unroll
+        for (int j = 0; j < BLK; j++) {
+            if (m0 + E * (lane + 64 * j) < K) {
+                const uint32_t wd[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
+#pragma unroll
+                for (int q = 0; q < E; q++) {
+                    const float wf = TYPE == T_F32 ? __uint_as_float(wd[q & 3])
+                                                   : f16_bits_to_f32((wd[q >> 1] >> (16 * (q & 1))) & 0xffffu);
+                    acc = fma((double)wf, (double)xv[j][q >> 2][q & 3], acc);   // exact product
+                }
+            }
+        }
+    }
+    const double t = wave_sum_f64(acc);
+    if (lane == 0) {
+        float v = (float)t;
+        if (a.add) v = addv + v;
+        a.y[(size_t)s * a.N + r] = v;
+    }
+}
+
 // One wave per row; lane l takes elements E*l + 64*E*i in order, the 64
 // partial sums meet in a fixed butterfly, so the result does not depend on
 // the grid.  SB streams (blockIdx.y selects the group of SB) share each
@@ -4793,7 +4840,7 @@ int kqk_launch_quantize_q8(const float* x, int K, int group, int8_t* xq, float* 
 
 // Dense rows (F16, F32): x staged in LDS when K <= DENSE_XLDS_MAX
 int kqk_launch_dense(int type, const void* w, const float* x, const float* add, float* y, int N,
-                     int K, int B, int grid, hipStream_t st) {
+                     int K, int B, int grid, int n_cu, hipStream_t st) {
     if ((type != T_F16 && type != T_F32) || N < 1 || K < 256 || (K & 255) || grid < 1 || B < 1 ||
         (B > 1 && add))
         return (int)hipErrorInvalidValue;
@@ -4801,6 +4848,12 @@ int kqk_launch_dense(int type, const void* w, const float* x, const float* add, 
     a.w = static_cast<const uint8_t*>(w);
     a.x = x; a.add = add; a.y = y; a.N = N; a.K = K; a.B = B;
     a.row_bytes = (long)K * (type == T_F32 ? 4 : 2);
+    if ((long)N * B <= (long)DENSE_FEW_WAVES * n_cu) {
+        const dim3 gf((N + 3) / 4, B);
+        if (type == T_F32) hipLaunchKernelGGL(kq_dense_few_kernel<T_F32>, gf, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL(kq_dense_few_kernel<T_F16>, gf, dim3(256), 0, st, a);
+        return (int)hipGetLastError();
+    }
     // DENSE_SB streams per wave share its weight loads, unless that leaves
     // fewer than 8 waves per CU (a 128-row MoE router at B = 16: 256 waves
     // of long serial chains); then one stream per wave

@@ -456,7 +456,7 @@ static int dense_gemv(int type, const void* w, const float* x, const float* add,
     if ((uintptr_t)w & 15) return kq_fail("dense GEMV: weights must be 16-byte aligned");
     long g = ((long)N + 3) / 4;
     if (g > 8L * g_kq.n_cu) g = 8L * g_kq.n_cu;
-    const int e = kqk_launch_dense(type, w, x, add, y, N, K, B, (int)g, st);
+    const int e = kqk_launch_dense(type, w, x, add, y, N, K, B, (int)g, g_kq.n_cu, st);
     if (e) return kq_fail("dense gemv launch: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }
