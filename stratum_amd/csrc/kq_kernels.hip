@@ -3109,18 +3109,11 @@ int launch_mfma_t(const float* x, const void* w, float* y, int B, int N, int K, 
 }
 
 // --------------------------------------------------------------- dequant
-// ------------------------------------------------- int8 MULTISEQ (MFMA)
-// st_linear_multix under g_st.use_sdot for Q4_K / Q6_K, B >= 2
-// (stratum_linear.h:732-907): every stream's x quantized as the
-// single-stream int8 mode quantizes it (kq_mi8_prep_kernel), then per
-// (row, stream) the reference's multix_pack arithmetic, bit for bit:
-//  Q4_K (q4k_dot_rows2_sdot_multix_pack, stratum_q4k_neon.h:870-948): per
-//    sub-block the binary32 term fl(fl(fl(d*sc) * fl(fl(L) * scl)) -
-//    fl(fl(dmin*m) * fl(fl(S) * scl))), added to a binary64 sum in element
-//    order (L the exact dot of the 4-bit values, S the group's int8 sum);
-//  Q6_K (q6k_dot_rows2_sdot_multix_pack, stratum_q6k_neon.h:627-700): per
-//    16-group ((double)d * sc * (double)scl) * (double)A in binary64, A the
-//    exact dot of q - 32.
+// ------------------------------------------------- int8 MoE batch (MFMA)
+// The runs of one expert's members in the int8 mode of Q4_K / Q6_K: every x
+// row quantized as the single-stream int8 mode quantizes it, then per (row,
+// member) the reference's multix_pack arithmetic, bit for bit (as in
+// kq_mi.hip, which holds the MULTISEQ call's own kernel).
 // The integer dots run on the matrix cores (v_mfma_i32_16x16x64_i8, exact
 // in int32), the terms and the sequential binary64 sums on the VALU.
 //
@@ -3137,38 +3130,26 @@ int launch_mfma_t(const float* x, const void* w, float* y, int B, int N, int K, 
 // D[i][j] lands in lane j + 16 (i/4), register i % 4: a lane holds its
 // weight row's dots for 2 streams x 2 sub-blocks (Q4_K) or 1 stream x 4
 // runs (Q6_K), in the order its binary64 sums need them.
-//
-// Work.  A wave owns 16 rows and SW streams for the whole row (the sums are
-// sequential in k); a workgroup's 4 waves take 4 neighbouring row blocks
-// with the same streams, whose quantized x and coefficients for one
-// super-block are staged in LDS (double-buffered, one barrier per
-// super-block) and read by all four.  Weights and staging data are loaded
-// P super-blocks ahead into registers: the x, coefficient and weight loads
-// of a super-block are issued together, so the in-order wait for one never
-// waits on data needed later.
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 struct Mi8Arg {
-    const uint8_t* w;         // N rows of K weights (Q4_K / Q6_K blocks)
     const int8_t* xq;         // [B][K] quantized streams
     const uint8_t* zp;        // 64 zero bytes
     const uint8_t* cf;        // per (stream, group) coefficients: Q4_K float2
                               // {scl, fl(fl(S) * scl)} [B][K/32]; Q6_K double
                               // scl [B][K/16]
-    float* y;                 // y[s * y_stride + r]
     long y_stride;
-    int N, K, B;
-    // grouped launches (the int8 MoE batch): blockIdx.y is group g < *ng of
-    // the kq_moe_group_kernel records (runs of at most 8 members of one
-    // expert); member slot j reads quantized row xi[j] and writes row
-    // yi[j] of the group's y (stride y_stride); slots past M read row zrow
-    // (all zero).  w and y above are unused.
+    int N, K;
+    // blockIdx.y is group g < *ng of the kq_moe_group_kernel records (runs of
+    // at most 8 members of one expert); member slot j reads quantized row
+    // xi[j] and writes row yi[j] of the group's y; slots past M read row zrow
+    // (all zero).
     const MxGroup* groups;
     const int* ng;
     int zrow;
     int rbw;                  // 16-row blocks per workgroup (1 unless KS = 1)
-    const float2* sm;         // grouped: {scale, sum} per (row, group)
-    int pack2;                // grouped Q4_K: runs of two members on the VALU
+    const float2* sm;         // {scale, sum} per (row, group)
+    int pack2;                // Q4_K: runs of two members on the VALU
 };
 
 // x -> int8 per group (the single-stream rule, kq_quantize_kernel's) and
@@ -3217,16 +3198,9 @@ __device__ __forceinline__ void mi8_prep_one(long gid, const float* x, long x_st
     if (sm) sm[gid] = make_float2(scale, (float)sum);   // the single-stream form's {scale, sum}
 }
 
-template <int G>
-__global__ __launch_bounds__(256) void kq_mi8_prep_kernel(const float* x, long x_stride, int K,
-                                                          int B, int bpad, int8_t* xq,
-                                                          uint8_t* cf, uint8_t* zp, float2* sm) {
-    mi8_prep_one<G>((long)blockIdx.x * 256 + threadIdx.x, x, x_stride, K, B, bpad, xq, cf, zp, sm);
-}
-
 // The int8 MoE batch's set-up in one launch: workgroup 0 cuts the runs
 // (moe_group_body, as kq_moe_group_kernel), the others quantize the x rows
-// (256 groups each, as kq_mi8_prep_kernel).  256-lane workgroups: the
+// (256 groups each).  256-lane workgroups: the
 // quantizing is about 300 VALU instructions per group, so 1024-lane
 // workgroups (four waves per SIMD on a few CUs) made it the longer part.
 template <int G>
@@ -3414,7 +3388,7 @@ __device__ __forceinline__ void mi8_pack2_q4k(const Mi8Arg& A, const MxGroup* gp
 struct Mi8W4 { uint4 hd, qv[4]; };
 struct Mi8W6 { uint32_t l[4][5], h[4][5], s[5]; uint32_t d, sh; };
 
-// Shape of one launch: SW streams per wave (8 streams x 2 sub-blocks per
+// Shape of one launch: 8 members per wave (8 streams x 2 sub-blocks per
 // Q4_K MFMA, 4 streams x 4 runs per Q6_K MFMA), P super-blocks of loads in
 // flight, and a workgroup of KS waves on one 16-row block, one K-part each.
 // A wave needs no other wave until the end: its weights, its A operands
@@ -3428,20 +3402,19 @@ struct Mi8W6 { uint32_t l[4][5], h[4][5], s[5]; uint32_t d, sh; };
 // the reference's strictly sequential sum unless a binary64 re-association
 // crosses a binary32 rounding boundary).
 //
-// GR (the int8 MoE batch, moe_forward_b under use_sdot,
-// stratum_arch_moe.inc.c:1158-1201): one workgroup per (16-row block, run of
+// moe_forward_b under use_sdot (stratum_arch_moe.inc.c:1158-1201): one workgroup per (16-row block, run of
 // one expert's members).  A run of two or more members takes
 // st_linear_multix's pack arithmetic above, exactly as a kq_gemv_multix_dev
 // call on that expert's slice would.  A run of one member takes the
 // single-stream path (mi8_single): the member equals its
 // kq_gemv_dev(type | KQ_INT8_ACT) result bit for bit.
-// (Q4_K: four waves per SIMD asked of the register allocator, which the
-// 16-stream forms reach with the A operands and coefficients out of the ring;
-// Q6_K reaches three by itself, and asking for them makes it spill)
-template <int TYPE, int SW, int P, int KS, bool GR>
+// (Q4_K: four waves per SIMD asked of the register allocator, which it
+// reaches with the A operands and coefficients out of the ring; Q6_K reaches three by itself, and asking for them makes it spill)
+template <int TYPE, int P, int KS>
 __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(TYPE == T_Q4K_I8 ? 4 : 1)))
 void kq_mi8_kernel(Mi8Arg A) {
     constexpr bool Q4 = TYPE == T_Q4K_I8;
+    constexpr int SW = 8;                           // member slots
     constexpr int NM = Q4 ? SW / 8 : SW / 4;        // MFMAs per chunk
     constexpr int NACC = Q4 ? 2 * NM : NM;          // binary64 sums per lane
     constexpr int CB = Q4 ? 64 : 128;               // coefficient bytes per stream and super-block
@@ -3456,33 +3429,24 @@ void kq_mi8_kernel(Mi8Arg A) {
     const int q = lane >> 4, jr = lane & 15;
     const int N = A.N, K = A.K, nb = K >> 8;
     const int ng = Q4 ? K >> 5 : K >> 4;            // coefficient groups per stream
-    const int s0 = GR ? 0 : blockIdx.y * SW;
     // row blocks rb0 .. rb0 + nrw - 1 (one after the other; KS = 1 only)
     const int rbw = KS == 1 ? A.rbw : 1;
     const int rb0 = blockIdx.x * rbw, nrw = min(rbw, (N + 15) / 16 - rb0);
     constexpr int BB = Q4 ? 144 : 210;
-    const MxGroup* gp = nullptr;
-    int M = SW;
-    const uint8_t* wbase = A.w;
-    if constexpr (GR) {
-        gp = A.groups + blockIdx.y;               // read with the count (in bounds)
-        const int ngv = *A.ng;
-        M = gp->M;
-        wbase = gp->w;
-        if ((int)blockIdx.y >= ngv) return;       // uniform over the workgroup
-    }
+    const MxGroup* gp = A.groups + blockIdx.y;      // read with the count (in bounds)
+    const int ngv = *A.ng;
+    const int M = gp->M;
+    const uint8_t* wbase = gp->w;
+    if ((int)blockIdx.y >= ngv) return;             // uniform over the workgroup
     // quantized row of member slot j (0 .. SW-1)
-    auto xrow = [&](int j) -> long {
-        if constexpr (GR) return j < M ? gp->xi[j] : A.zrow;
-        return s0 + j;
-    };
-    if (GR && M == 1) {                           // uniform
+    auto xrow = [&](int j) -> long { return j < M ? gp->xi[j] : A.zrow; };
+    if (M == 1) {                                 // uniform
         extern __shared__ __align__(16) double mi8_terms[];
         mi8_single<TYPE>(A, wbase, gp->xi[0], gp->y + (size_t)gp->yi[0] * A.y_stride, rb0, nrw,
                          mi8_terms, tid, 64 * KS);
         return;
     }
-    if constexpr (GR && Q4 && KS == 1) {
+    if constexpr (Q4 && KS == 1) {
         if (M == 2 && A.pack2) {                  // uniform
             extern __shared__ __align__(16) double mi8_terms[];
             mi8_pack2_q4k(A, gp, rb0, nrw, reinterpret_cast<uint8_t*>(mi8_terms), tid);
@@ -3573,13 +3537,7 @@ void kq_mi8_kernel(Mi8Arg A) {
 #pragma unroll
         for (int a = 0; a < NACC; a++) {
             const int so = Q4 ? 8 * (a >> 1) + 2 * q + (a & 1) : 4 * a + q;   // member slot
-            if (r < N) {
-                if constexpr (GR) {
-                    if (so < M) gp->y[(size_t)gp->yi[so] * A.y_stride + r] = (float)acc[a];
-                } else if (s0 + so < A.B) {
-                    A.y[(size_t)(s0 + so) * A.y_stride + r] = (float)acc[a];
-                }
-            }
+            if (r < N && so < M) gp->y[(size_t)gp->yi[so] * A.y_stride + r] = (float)acc[a];
             acc[a] = 0.0;
         }
     };
@@ -4884,8 +4842,8 @@ int kqk_mi8_parts(int K) {
     return nb >= 48 ? 4 : nb >= 12 ? 2 : 1;
 }
 
-// (streams padded to a multiple of 16, the widest wave's stream count)
-long kqk_mi8_workspace(int type, int B, int K, long* cf_off) {
+// (rows padded to a multiple of 16)
+static long mi8_workspace(int type, int B, int K, long* cf_off) {
     if ((type != T_Q4K_I8 && type != T_Q6K_I8) || B < 1 || K < 256 || (K & 255)) return -1;
     const long bp = (B + 15) & ~15L;
     const long xb = (bp * K + 255) & ~255L;
@@ -4894,77 +4852,12 @@ long kqk_mi8_workspace(int type, int B, int K, long* cf_off) {
     return xb + ((cb + 255) & ~255L) + 256;     // + the zero page
 }
 
-int kqk_launch_mi8(int type, const float* xs, long x_stride, const void* w, float* ys,
-                   long y_stride, int B, int N, int K, void* ws, int ks, hipStream_t st) {
-    long cf_off = 0;
-    const long wsb = kqk_mi8_workspace(type, B, K, &cf_off);
-    if (wsb < 0 || N < 1 || B < 2 || (x_stride & 3) || x_stride < K || y_stride < N ||
-        ((uintptr_t)xs & 15) || ((uintptr_t)ws & 255))
-        return (int)hipErrorInvalidValue;
-    int8_t* xq = static_cast<int8_t*>(ws);
-    uint8_t* cf = static_cast<uint8_t*>(ws) + cf_off;
-    uint8_t* zp = static_cast<uint8_t*>(ws) + wsb - 256;   // zeroed by the prep kernel
-    const int G = type == T_Q4K_I8 ? 32 : 16;
-    const int bpad = (B + 15) & ~15;
-    const long groups = (long)bpad * (K / G);
-    if (G == 32)
-        hipLaunchKernelGGL(kq_mi8_prep_kernel<32>, dim3((unsigned)((groups + 255) / 256)), dim3(256),
-                           0, st, xs, x_stride, K, B, bpad, xq, cf, zp, nullptr);
-    else
-        hipLaunchKernelGGL(kq_mi8_prep_kernel<16>, dim3((unsigned)((groups + 255) / 256)), dim3(256),
-                           0, st, xs, x_stride, K, B, bpad, xq, cf, zp, nullptr);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
-    Mi8Arg a;
-    a.w = static_cast<const uint8_t*>(w);
-    a.xq = xq;
-    a.zp = zp;
-    a.cf = cf;
-    a.y = ys;
-    a.y_stride = y_stride;
-    a.N = N; a.K = K; a.B = B;
-    a.groups = nullptr; a.ng = nullptr; a.zrow = 0; a.rbw = 1; a.sm = nullptr; a.pack2 = 0;
-    // Q4_K: 8 or 16 streams per wave; Q6_K: 8 (its A operands take
-    // 16 registers per MFMA and super-block)
-    // (8 streams per wave up to B = 8, one super-block in flight; measured
-    // at the 27B gate, B = 8 .. 64, against 8 streams at every B and two
-    // super-blocks in flight)
-#ifndef KQ_MI8_SWB
-#define KQ_MI8_SWB 8
-#endif
-#ifndef KQ_MI8_P8
-#define KQ_MI8_P8 1
-#endif
-    const int SW = type == T_Q6K_I8 || B <= KQ_MI8_SWB ? 8 : 16;
-    const int nset = (B + SW - 1) / SW, nrb = (N + 15) / 16;
-    // K-parts: a function of the row length only (kqk_mi8_parts), so the
-    // binary64 grouping -- and with it the result -- does not depend on the
-    // batch or the row count
-    if (ks != 1 && ks != 2 && ks != 4 && ks != 8) ks = kqk_mi8_parts(K);
-#define KQ_MI8_GO(T_, S_, P_, K_)                                                            \
-    hipLaunchKernelGGL((kq_mi8_kernel<T_, S_, P_, K_, false>), dim3((unsigned)nrb,           \
-                       (unsigned)nset), dim3(64 * K_), 0, st, a)
-#define KQ_MI8_KS(T_, S_, P_)                                                                \
-    if (ks == 1) KQ_MI8_GO(T_, S_, P_, 1);                                                   \
-    else if (ks == 2) KQ_MI8_GO(T_, S_, P_, 2);                                              \
-    else if (ks == 4) KQ_MI8_GO(T_, S_, P_, 4);                                              \
-    else KQ_MI8_GO(T_, S_, P_, 8);
-    if (type == T_Q4K_I8) {
-        if (SW == 8) { KQ_MI8_KS(T_Q4K_I8, 8, KQ_MI8_P8) } else { KQ_MI8_KS(T_Q4K_I8, 16, 1) }
-    } else {
-        KQ_MI8_KS(T_Q6K_I8, 8, 1)
-    }
-#undef KQ_MI8_KS
-#undef KQ_MI8_GO
-    return (int)hipGetLastError();
-}
-
 // The int8 MoE batch: workspace bytes for nx quantized x rows (plus the
 // zero row: the MULTISEQ workspace of nx + 1 streams, then the rows'
 // {scale, sum} pairs) and the launches: the runs of at most 8 members of
 // one expert (kq_moe_group_kernel's rule; records in groups, their count
 // in *ng, at most ngmax) together with the quantized x rows (nx = nm /
-// x_div of them), then the grouped main kernel.  K-parts as kqk_launch_mi8
+// x_div of them), then the grouped main kernel.  K-parts as kqk_launch_mi
 // takes them, so a run's members equal a kq_gemv_multix_dev call over them.
 #ifndef KQ_MI8_RBW
 #define KQ_MI8_RBW 2
@@ -4976,7 +4869,7 @@ int kqk_launch_mi8(int type, const float* xs, long x_stride, const void* w, floa
 #define KQ_MI8G_P 1
 #endif
 static long mi8_moe_layout(int type, int nx, int K, long* cf_off, long* sm_off, long* zp_off) {
-    const long base = nx < 1 ? -1 : kqk_mi8_workspace(type, nx + 1, K, cf_off);
+    const long base = nx < 1 ? -1 : mi8_workspace(type, nx + 1, K, cf_off);
     if (base < 0) return -1;
     const long bpad = (nx + 1 + 15) & ~15L;
     *zp_off = base - 256;
@@ -5049,11 +4942,9 @@ int kqk_launch_mi8_moe(int type, const int* sel, int nm, int E, int nt, int x_di
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     Mi8Arg a;
-    a.w = nullptr;
     a.xq = xq; a.zp = zp; a.cf = cf;
-    a.y = nullptr;
     a.y_stride = y_stride;
-    a.N = N; a.K = K; a.B = 8;
+    a.N = N; a.K = K;
     a.groups = static_cast<const MxGroup*>(groups);
     a.ng = ng;
     a.zrow = nx;
@@ -5062,7 +4953,7 @@ int kqk_launch_mi8_moe(int type, const int* sel, int nm, int E, int nt, int x_di
     a.pack2 = pack2;
     const int nrb = ((N + 15) / 16 + rbw - 1) / rbw;
 #define KQ_MI8G_GO(T_, P_, K_)                                                               \
-    hipLaunchKernelGGL((kq_mi8_kernel<T_, 8, P_, K_, true>), dim3((unsigned)nrb,             \
+    hipLaunchKernelGGL((kq_mi8_kernel<T_, P_, K_>), dim3((unsigned)nrb,             \
                        (unsigned)ngmax), dim3(64 * K_), (size_t)tl, st, a)
 #define KQ_MI8G_KS(T_, P_)                                                                   \
     if (ks == 1) KQ_MI8G_GO(T_, P_, 1);                                                      \

@@ -220,7 +220,8 @@ static int kq_ready(void) {
     g_kq.n_cu = ncu > 0 ? ncu : 1;
     g_kq.lds_max = lds > 0 ? lds : 65536;
     if (kqk_set_max_lds(g_kq.lds_max) != 0 || kqk_mx_set_max_lds(g_kq.lds_max) != 0 ||
-        kqk_dense_set_max_lds(g_kq.lds_max) != 0 || kqk_mv_set_max_lds(g_kq.lds_max) != 0)
+        kqk_dense_set_max_lds(g_kq.lds_max) != 0 || kqk_mv_set_max_lds(g_kq.lds_max) != 0 ||
+        kqk_mi_set_max_lds(g_kq.lds_max) != 0)
         return kq_fail("cannot raise the LDS limit");
     /* the static scratch of the no-allocation entry point: its address on
      * this device, looked up once now (other devices at their first call) */
@@ -646,12 +647,11 @@ static int mfma_reserve(kq_scr* sc, size_t need);
  * reference's multix_pack arithmetic. */
 static int mi8_multix(int type, const void* w, const float* xs, float* ys, int B, int N, int K,
                       hipStream_t st) {
-    long cf_off = 0;
-    const long need = kqk_mi8_workspace(type, B, K, &cf_off);
+    const long need = kqk_mi_workspace(type, B, K);
     if (need < 0) return kq_fail("int8 multix: bad shape B=%d K=%d", B, K);
     kq_scr* sc = scr_of(st);
     if (!sc || mfma_reserve(sc, (size_t)need)) return -1;
-    const int e = kqk_launch_mi8(type, xs, K, w, ys, N, B, N, K, sc->mf, 0, st);
+    const int e = kqk_launch_mi(type, xs, K, w, ys, N, B, N, K, sc->mf, st);
     if (e) return kq_fail("int8 multix launch: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }
@@ -1278,7 +1278,7 @@ static size_t moe_i8_bytes(int type, int nx, int K, int nt, int nm, int E) {
  * arithmetic, a ticket of one the single-stream path.  Here the same runs
  * are cut on the device (kq_moe_group_kernel's rule, run length 8) in the
  * launch that quantizes every x row once, and one grouped matrix-core
- * launch computes all runs (kq_mi8_kernel, GR): each member equals
+ * launch computes all runs (kq_mi8_kernel): each member equals
  * kq_gemv_multix_dev over its run (kq_gemv_dev for a run of one) bit for
  * bit.  (For Q5_K, Q3_K and Q8_0 st_linear_multix is per stream -- Q8_0's
  * pack equals its single-stream path, stratum_q8_0.h:145-149 -- so the
