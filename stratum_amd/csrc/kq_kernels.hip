@@ -4026,6 +4026,13 @@ __global__ __launch_bounds__(256) void kq_softmax_kernel(float* x, int E) {
     for (int i = tid; i < E; i += 256) row[i] = sm[i] * inv;
 }
 
+// n4 float4 between pinned host memory and the device, one per lane: bounded
+// by the round trip over PCIe, which every load of the launch shares.
+__global__ __launch_bounds__(256) void kq_copy_kernel(const float4* s, float4* d, int n4) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) d[i] = s[i];
+}
+
 // SwiGLU (stratum_swiglu, stratum_engine.h:373-392, the scalar loop):
 // y = (g / (1 + expf(-g))) * u, binary32 throughout, 4 values per lane.
 __global__ __launch_bounds__(256) void kq_swiglu_kernel(const float* g, const float* u, float* y,
@@ -4764,6 +4771,15 @@ int kqk_launch_softmax(float* x, int B, int E, hipStream_t st) {
     if (B < 1 || E < 1 || E > KQ_MOE_MAX_EXPERTS) return (int)hipErrorInvalidValue;
     const size_t shm = (size_t)(((E + 3) & ~3) + 64) * sizeof(float);
     hipLaunchKernelGGL(kq_softmax_kernel, dim3(B), dim3(256), shm, st, x, E);
+    return (int)hipGetLastError();
+}
+
+// (both 16-byte aligned, with room for whole float4s)
+int kqk_launch_copy(const float* src, float* dst, long n, hipStream_t st) {
+    const long n4 = (n + 3) / 4;
+    if (n < 1 || n4 > (1L << 30)) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(kq_copy_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st,
+                       reinterpret_cast<const float4*>(src), reinterpret_cast<float4*>(dst), (int)n4);
     return (int)hipGetLastError();
 }
 

@@ -52,6 +52,7 @@ int kqk_launch_dense(int type, const void* w, const float* x, const float* add, 
 int kqk_launch_q2k_to_nib(const void* q2k, void* nib, long nblocks, hipStream_t st);
 /* MoE FFN step pieces */
 int kqk_launch_softmax(float* x, int B, int E, hipStream_t st);
+int kqk_launch_copy(const float* src, float* dst, long n, hipStream_t st);
 int kqk_launch_swiglu(const float* g, const float* u, float* y, long n, hipStream_t st);
 int kqk_launch_moe_combine(const float* o, const int* sel, const float* selw, const float* resid,
                            float* x, int B, int k, int H, hipStream_t st);

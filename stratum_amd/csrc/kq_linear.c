@@ -59,6 +59,8 @@ typedef struct {
     float* d_x; size_t cap_x;
     float* d_y; size_t cap_y;
     float* d_a; size_t cap_a;
+    float* io;             /* pinned: KQ_IO_FLOATS in, KQ_IO_FLOATS out */
+    float* io_dev;         /* its device address */
     kq_scr scr[KQ_SCR_SLOTS];       /* the device entries' scratch, per stream */
     unsigned long long scr_calls;   /* scr_of calls, for the least recently used */
     size_t mf_reserve;              /* kq_reserve_mfma_workspace: least mf size */
@@ -298,6 +300,7 @@ void kq_linear_shutdown(void) {
     if (g_kq.d_x) (void)hipFree(g_kq.d_x);
     if (g_kq.d_y) (void)hipFree(g_kq.d_y);
     if (g_kq.d_a) (void)hipFree(g_kq.d_a);
+    if (g_kq.io) (void)hipHostFree(g_kq.io);
     for (int i = 0; i < KQ_SCR_SLOTS; i++) {
         if (g_kq.scr[i].moe) (void)hipFree(g_kq.scr[i].moe);
         if (g_kq.scr[i].mf) (void)hipFree(g_kq.scr[i].mf);
@@ -311,7 +314,7 @@ static int grow(float** p, size_t* cap, size_t nfloats) {
     if (*p) (void)hipFree(*p);
     *p = NULL;
     *cap = 0;
-    size_t n = nfloats < 4096 ? 4096 : nfloats;
+    size_t n = nfloats < 4096 ? 4096 : (nfloats + 3) & ~(size_t)3;   /* whole float4s */
     if (hip_ok(hipMalloc((void**)p, n * sizeof(float)), "hipMalloc(staging)")) return -1;
     *cap = n;
     return 0;
@@ -850,15 +853,73 @@ int kq_quantize_x_q8_dev(const float* x, int K, int group, int8_t* xq, float* xs
     return 0;
 }
 
-static int h2d(float* d, const float* h, size_t n) {
-    return hip_ok(hipMemcpyAsync(d, h, n * sizeof(float), hipMemcpyHostToDevice, g_kq.stream),
+/* Host x and y.  hipMemcpyAsync from memory that is not pinned goes through
+ * the runtime's own buffers and waits there: about 5 us a vector in and out.
+ * Up to KQ_IO_FLOATS a direction, the host copies x to pinned memory, from
+ * where a kernel moves it to the device (each workgroup of the product reads
+ * all of x: too much for PCIe), and the product writes its y, which it stores
+ * once, to pinned memory itself (a copy launch of its own in its place: 1 to
+ * 2 us more at every size tried, N = 32 to 60000).  Longer vectors are copied
+ * as they are: the buffer's bound.  Q4_K 1024 x 1024 26.8 -> 18.0 us, 17408 x
+ * 5120 41.6 -> 28.8, eight streams of 1024 x 1024 160 -> 23.7. */
+#define KQ_IO_FLOATS 65536
+
+static int io_ready(void) {
+    if (g_kq.io) return 1;
+    if (hipHostMalloc((void**)&g_kq.io, 2 * KQ_IO_FLOATS * sizeof(float), hipHostMallocDefault) ==
+        hipSuccess) {
+        if (hipHostGetDevicePointer((void**)&g_kq.io_dev, g_kq.io, 0) == hipSuccess) return 1;
+        (void)hipHostFree(g_kq.io);
+    }
+    (void)hipGetLastError();
+    g_kq.io = NULL;
+    return 0;
+}
+
+/* B vectors of n floats to d, one after the other; off: floats of the pinned
+ * buffer that this call has used */
+static int h2d(float* d, const float* const* hs, int B, size_t n, size_t off) {
+    for (int s = 0; s < B; s++)
+        if (!hs[s]) return kq_fail("copy x in: NULL pointer");
+    off = (off + 3) & ~(size_t)3;
+    if (off + (size_t)B * n > KQ_IO_FLOATS || !io_ready()) {
+        for (int s = 0; s < B; s++)
+            if (hip_ok(hipMemcpyAsync(d + (size_t)s * n, hs[s], n * sizeof(float),
+                                      hipMemcpyHostToDevice, g_kq.stream), "copy x in"))
+                return -1;
+        return 0;
+    }
+    for (int s = 0; s < B; s++) memcpy(g_kq.io + off + (size_t)s * n, hs[s], n * sizeof(float));
+    return hip_ok((hipError_t)kqk_launch_copy(g_kq.io_dev + off, d, (long)((size_t)B * n), g_kq.stream),
                   "copy x in");
 }
 
-static int finish_y(float* y, const float* d_y, size_t n) {
-    if (hip_ok(hipMemcpyAsync(y, d_y, n * sizeof(float), hipMemcpyDeviceToHost, g_kq.stream),
-               "copy y out")) return -1;
-    return hip_ok(hipStreamSynchronize(g_kq.stream), "synchronize");
+/* where a call's y of n floats goes on the device */
+static float* y_dev(size_t n) {
+    return n <= KQ_IO_FLOATS && io_ready() ? g_kq.io_dev + KQ_IO_FLOATS : g_kq.d_y;
+}
+
+/* y[0 .. B-1] of ns[s] floats (ns NULL: n each) from d = y_dev, one after the
+ * other, and the wait for them */
+static int finish_y(float* const* ys, const int* ns, int n, int B, const float* d) {
+    const int pin = d != g_kq.d_y;
+    for (int s = 0; s < B; s++)
+        if (!ys[s]) return kq_fail("copy y out: NULL pointer");
+    size_t off = 0;
+    for (int s = 0; s < B && !pin; s++) {
+        const size_t m = (size_t)(ns ? ns[s] : n);
+        if (hip_ok(hipMemcpyAsync(ys[s], d + off, m * sizeof(float), hipMemcpyDeviceToHost,
+                                  g_kq.stream), "copy y out"))
+            return -1;
+        off += m;
+    }
+    if (hip_ok(hipStreamSynchronize(g_kq.stream), "synchronize")) return -1;
+    for (int s = 0; s < B && pin; s++) {
+        const size_t m = (size_t)(ns ? ns[s] : n);
+        memcpy(ys[s], g_kq.io + KQ_IO_FLOATS + off, m * sizeof(float));
+        off += m;
+    }
+    return 0;
 }
 
 int kq_linear_dispatch_add(const kq_tensor* w, const float* x, const float* add,
@@ -869,15 +930,16 @@ int kq_linear_dispatch_add(const kq_tensor* w, const float* x, const float* add,
     if (!dw) return -1;
     if (grow(&g_kq.d_x, &g_kq.cap_x, (size_t)K) || grow(&g_kq.d_y, &g_kq.cap_y, (size_t)N))
         return -1;
-    if (h2d(g_kq.d_x, x, (size_t)K)) return -1;
+    if (h2d(g_kq.d_x, &x, 1, (size_t)K, 0)) return -1;
     const float* d_add = NULL;
     if (add) {
-        if (grow(&g_kq.d_a, &g_kq.cap_a, (size_t)N) || h2d(g_kq.d_a, add, (size_t)N)) return -1;
+        if (grow(&g_kq.d_a, &g_kq.cap_a, (size_t)N) || h2d(g_kq.d_a, &add, 1, (size_t)N, (size_t)K))
+            return -1;
         d_add = g_kq.d_a;
     }
-    if (kq_gemv_dev(sdot_type((int)w->type), dw, g_kq.d_x, d_add, g_kq.d_y, N, K, g_kq.stream))
-        return -1;
-    return finish_y(y, g_kq.d_y, (size_t)N);
+    float* dy = y_dev((size_t)N);
+    if (kq_gemv_dev(sdot_type((int)w->type), dw, g_kq.d_x, d_add, dy, N, K, g_kq.stream)) return -1;
+    return finish_y(&y, NULL, N, 1, dy);
 }
 
 int kq_linear_dispatch(const kq_tensor* w, const float* x, float* y, int N, int K) {
@@ -893,15 +955,11 @@ int kq_linear_multix(const kq_tensor* w, const float* const* xs, float* const* y
     if (!dw) return -1;
     if (grow(&g_kq.d_x, &g_kq.cap_x, (size_t)B * K) ||
         grow(&g_kq.d_y, &g_kq.cap_y, (size_t)B * N)) return -1;
-    for (int s = 0; s < B; s++)
-        if (h2d(g_kq.d_x + (size_t)s * K, xs[s], (size_t)K)) return -1;
-    if (kq_gemv_multix_dev(sdot_type((int)w->type), dw, g_kq.d_x, g_kq.d_y, B, N, K, g_kq.stream))
+    if (h2d(g_kq.d_x, xs, B, (size_t)K, 0)) return -1;
+    float* dy = y_dev((size_t)B * N);
+    if (kq_gemv_multix_dev(sdot_type((int)w->type), dw, g_kq.d_x, dy, B, N, K, g_kq.stream))
         return -1;
-    for (int s = 0; s < B; s++)
-        if (hip_ok(hipMemcpyAsync(ys[s], g_kq.d_y + (size_t)s * N, (size_t)N * sizeof(float),
-                                  hipMemcpyDeviceToHost, g_kq.stream), "copy y out"))
-            return -1;
-    return hip_ok(hipStreamSynchronize(g_kq.stream), "synchronize");
+    return finish_y(ys, NULL, N, B, dy);
 }
 
 int kq_q4k_group(const float* x, int K,
@@ -926,22 +984,16 @@ int kq_q4k_group(const float* x, int K,
         ytot += (size_t)Ns[i];
     }
     if (grow(&g_kq.d_x, &g_kq.cap_x, (size_t)K) || grow(&g_kq.d_y, &g_kq.cap_y, ytot)) return -1;
-    if (h2d(g_kq.d_x, x, (size_t)K)) return -1;
+    if (h2d(g_kq.d_x, &x, 1, (size_t)K, 0)) return -1;
+    float* dy = y_dev(ytot);
     size_t off = 0;
     for (int i = 0; i < nw; i++) {
         sg[i].x = g_kq.d_x;
-        sg[i].y = g_kq.d_y + off;
+        sg[i].y = dy + off;
         off += (size_t)Ns[i];
     }
     if (kq_gemv_segments_dev(sg, nw, g_kq.stream)) return -1;
-    off = 0;
-    for (int i = 0; i < nw; i++) {
-        if (hip_ok(hipMemcpyAsync(ys[i], g_kq.d_y + off, (size_t)Ns[i] * sizeof(float),
-                                  hipMemcpyDeviceToHost, g_kq.stream), "copy y out"))
-            return -1;
-        off += (size_t)Ns[i];
-    }
-    return hip_ok(hipStreamSynchronize(g_kq.stream), "synchronize");
+    return finish_y(ys, Ns, 0, nw, dy);
 }
 
 /* ------------------------------------------------------------ MoE gather */
