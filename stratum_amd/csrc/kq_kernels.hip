@@ -2582,9 +2582,18 @@ __global__ __launch_bounds__(1024) void kq_moe_group_kernel(MoeGroupArg a) {
 //    workgroup sweeps a block of 256 (Q4_K) or 128 (Q6_K) rows.  The
 //    (row block, super-block) iterations are split into one contiguous range
 //    per workgroup (whole row blocks when there are at least two per
-//    workgroup); a super-block's planes for all stream groups are staged in
-//    LDS (double-buffered) while the previous super-block is consumed, and
-//    each weight step is decoded once for every stream group;
+//    workgroup); each weight step is decoded once for every stream group.
+//    All loads go straight to LDS in address order (global_load_lds), an
+//    iteration ahead: the planes in half stages (a ring of three: with
+//    Q4_K's weights two whole stages of 64 streams pass 160 KB), the weights
+//    in each wave's own place, which is free once the wave has read its
+//    block.  With the weights loaded one row per lane to registers every
+//    lane of a load was a cache access of its own, and the planes took
+//    registers and LDS stores on the way.  Measured against that, with the
+//    split and the reduction, B = 16 / 32 / 48 / 64: 17408 x 5120 Q4_K 29.4 /
+//    35.8 / 43.5 / 51.1 -> 27.4 / 34.4 / 41.3 / 48.6 us; 5120 x 17408 Q6_K
+//    47.8 / 52.1 / 59.8 / 68.7 -> 39.2 / 46.2 / 55.9 / 64.3 us; 1000 x 1024
+//    Q6_K B = 16 12.3 -> 10.7 us, the same results bit for bit;
 //  * kq_mf_reduce_kernel adds, in workgroup order, the partial sums of the
 //    row blocks that several workgroups share (a fixed order: the result
 //    does not depend on timing).
@@ -2598,9 +2607,6 @@ template <int TYPE> struct MfShape {
     static constexpr int TILES = TYPE == T_Q4K ? 2 : 1;
     static constexpr int ROWS = 16 * TILES * MF_NW;                    // rows per row block
 };
-
-// uint4 of one super-block's LDS stage for nsg stream groups
-__host__ __device__ constexpr int mf_stage_u4(int nsg) { return nsg * (MF_GROUP_U4 + MF_SIDE_U4); }
 
 // How the (row block, super-block) iterations go to the workgroups: whole
 // row blocks per workgroup when there are at least two per workgroup, else
@@ -2701,6 +2707,7 @@ struct MfArg {
     float* y;                // B x N
     float* part;             // (G + nrb) slots x 16 NSG x rows: partial sums
     int B, N, K, NSG, nrb, G, whole;
+    int walign;              // weights 16-byte aligned
     long T;
 };
 
@@ -2717,54 +2724,41 @@ template <> struct MfRaw<T_Q4K> { using T = MfRawQ4; };
 template <> struct MfRaw<T_Q6K> { using T = MfRawQ6; };
 
 // Q4_K: chunk c's 8 bytes for this lane: low nibbles are sub-block 2c at
-// positions 64c + 8kg + v, high nibbles sub-block 2c + 1 at 64c + 32 + 8kg + v
-__device__ __forceinline__ MfRawQ4 mf_load_q4k(wptr blk, int kg) {
+// positions 64c + 8kg + v, high nibbles sub-block 2c + 1 at 64c + 32 + 8kg + v.
+// wl: the wave's weights in LDS, 144 bytes a row
+__device__ __forceinline__ MfRawQ4 mf_read_q4k(const uint8_t* wl, int r16, int kg) {
     MfRawQ4 r;
-    r.hd = ld16(blk);
+    const uint8_t* blk = wl + 144 * r16;
+    r.hd = *reinterpret_cast<const uint4*>(blk);
 #pragma unroll
-    for (int c = 0; c < 4; c++) r.q[c] = ld8a4(blk + 16 + 32 * c + 8 * kg);
+    for (int c = 0; c < 4; c++) r.q[c] = *reinterpret_cast<const uint2*>(blk + 16 + 32 * c + 8 * kg);
     return r;
 }
 
 // Q6_K: positions 32 st + 8 kg + v (step st = 4h + t) are bytes
 // 64h + 32(t&1) + 16(kg>>1) + 8(kg&1) + v of ql (nibble t >> 1) and
 // 128 + 32h + 16(kg>>1) + 8(kg&1) + v of qh (bits 2t): four ql fields and
-// two qh fields of 8 bytes, each read as three dwords of the 4-aligned
-// block and realigned (the third repeats the second when the block is
-// aligned, so no read passes the block's 210 bytes); the lane's sub-block
-// scales are bytes 192 + 2 st + (kg >> 1).
-__device__ __forceinline__ MfRawQ6 mf_load_q6k(wptr blk, int kg) {
+// two qh fields of 8 bytes, each read as three dwords and realigned (the row
+// lies in LDS as the 55 dwords from the one that holds its first byte, which
+// is bits sh of it); the lane's sub-block scales are bytes 192 + 2 st + (kg >> 1).
+__device__ __forceinline__ MfRawQ6 mf_read_q6k(const uint8_t* wl, int r16, int kg, uint32_t sh) {
     MfRawQ6 r;
-    const uint32_t mis = (uint32_t)reinterpret_cast<uintptr_t>(blk) & 3u;
-    r.sh = mis * 8u;
-    const wptr b4 = blk - mis;
-    const int nx = mis ? 4 : 0;
-    const int o = 16 * (kg >> 1) + 8 * (kg & 1);
+    r.sh = sh;
+    const uint8_t* blk = wl + 220 * r16;
+    auto dw = [&](int o) { return *reinterpret_cast<const uint32_t*>(blk + o); };
+    const int o = 8 * kg;
 #pragma unroll
-    for (int f = 0; f < 4; f++) {
-        const int off = 64 * (f >> 1) + 32 * (f & 1) + o;
-        r.ql[f][0] = ld4(b4 + off);
-        r.ql[f][1] = ld4(b4 + off + 4);
-        r.ql[f][2] = ld4(b4 + off + 4 + nx);
-    }
+    for (int f = 0; f < 4; f++)
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int off = 128 + 32 * h + o;
-        r.qh[h][0] = ld4(b4 + off);
-        r.qh[h][1] = ld4(b4 + off + 4);
-        r.qh[h][2] = ld4(b4 + off + 4 + nx);
-    }
-    const uint4 sv = ld16a4(b4 + 192);
-    r.sc[0] = sv.x; r.sc[1] = sv.y; r.sc[2] = sv.z; r.sc[3] = sv.w;
-    r.sc[4] = ld4(b4 + 192 + 12 + nx);
-    r.d = ld2(blk + 208);
+        for (int k = 0; k < 3; k++) r.ql[f][k] = dw(64 * (f >> 1) + 32 * (f & 1) + o + 4 * k);
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) r.qh[h][k] = dw(128 + 32 * h + o + 4 * k);
+#pragma unroll
+    for (int k = 0; k < 5; k++) r.sc[k] = dw(192 + 4 * k);
+    r.d = __builtin_amdgcn_alignbit(dw(212), dw(208), sh) & 0xffffu;
     return r;
-}
-
-template <int TYPE>
-__device__ __forceinline__ typename MfRaw<TYPE>::T mf_load(wptr blk, int kg) {
-    if constexpr (TYPE == T_Q4K) return mf_load_q4k(blk, kg);
-    else return mf_load_q6k(blk, kg);
 }
 
 // fp16 of sc * q for the 4 nibble bytes of nib (each < 16), sc <= 63: the
@@ -2868,18 +2862,44 @@ __device__ __forceinline__ void mf_step_q6k(const MfRawQ6& r, const MfSb<T_Q6K>&
     wl = __builtin_bit_cast(half8, make_uint4(l4[0], l4[1], l4[2], l4[3]));
 }
 
+// LDS of kq_mf_kernel: three half stages of planes, two of x sums and E, and
+// each wave's weight blocks (Q4_K 16-byte pieces, Q6_K 55 dwords a row)
+template <int TYPE> constexpr int mf_wb() { return TYPE == T_Q4K ? 2 * 16 * 144 : 14 * 256; }
+template <int TYPE> constexpr size_t mf_lds(int nsg) {
+    return 3 * (size_t)nsg * (MF_GROUP_U4 / 2) * 16 + 2 * (size_t)nsg * MF_SIDE_U4 * 16 +
+           (size_t)MF_NW * mf_wb<TYPE>();
+}
+
+// One 64-lane load straight to LDS: lane i's bytes go to dst + 16 i (4 i);
+// dst and src uniform
+__device__ __forceinline__ void mf_glds16(uint32_t dst, uint32_t off, const void* src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(src) : "memory");
+}
+__device__ __forceinline__ void mf_glds4(uint32_t dst, uint32_t off, const void* src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(src) : "memory");
+}
+// at most N loads of this wave outstanding, its LDS reads done, then a barrier
+// that leaves those loads in flight
+template <int N> __device__ __forceinline__ void mf_wait_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+}
+
 template <int TYPE, int NSG>
 __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
     using TI = TypeInfo<TYPE>;
     using SH = MfShape<TYPE>;
-    constexpr int TL = SH::TILES, R = SH::ROWS, NT = 64 * MF_NW;
-    constexpr int PU = NSG * MF_GROUP_U4, NX = NSG * MF_SIDE_U4, SU = PU + NX;   // uint4 per stage
-    constexpr int NP = PU / NT;                                        // plane uint4 per thread
-    constexpr int NH = NP / 2 + 1;                                     // per staging half
-    static_assert(NP * NT == PU && NP % 2 == 0 && NX <= NT, "stage split");
+    constexpr bool Q4 = TYPE == T_Q4K;
+    constexpr int TL = SH::TILES, R = SH::ROWS;
+    constexpr int PU = NSG * MF_GROUP_U4, NX = NSG * MF_SIDE_U4;       // uint4 per super-block
+    constexpr int HU = PU / 2;                                         // and per half stage
+    constexpr int SIDE = 3 * HU * 16, WL = SIDE + 2 * NX * 16, WB = mf_wb<TYPE>();   // LDS bytes
     extern __shared__ __align__(16) uint8_t smem[];
-    u32x4* lds = reinterpret_cast<u32x4*>(smem);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kg = lane >> 4;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(uint8_t __attribute__((address_space(3)))*)smem;
+    const u32x4* lds = reinterpret_cast<const u32x4*>(smem);
+    const int tid = threadIdx.x, lane = tid & 63, kg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int NSB = A.K >> 8;
     const size_t rbytes = (size_t)NSB * TI::BB;
     const int wg = blockIdx.x;
@@ -2892,72 +2912,116 @@ __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
         it1 = (int)((long)(wg + 1) * A.T / A.G);
     }
     if (it0 >= it1) return;                 // the whole workgroup: no barrier is left waiting
-    auto wrow = [&](int rb, int t) {
-        const int row = rb * R + 16 * (TL * wave + t) + (lane & 15);
-        return to_global(A.w) + (size_t)min(row, A.N - 1) * rbytes;
-    };
-    // staging of super-block sb in two halves (the planes' first half; the
-    // second half, the x sums and E); the loads are branch-free (clamped), so
-    // the compiler counts outstanding loads exactly
-    auto sload = [&](int h, int sb, u32x4 (&v)[NH]) {
-        const u32x4* pp = reinterpret_cast<const u32x4*>(A.planes) + (size_t)sb * PU + tid + NT * (NP / 2) * h;
+
+    // Loads of one iteration, all straight to LDS, in this order a wave: NW of
+    // its weights (rows of 16 TL, in address order), one of the x sums and E,
+    // NSG of the planes' first half (steps 0-3 of every group), and, half an
+    // iteration later, NSG of the second half.
+    constexpr int NW = Q4 ? 5 : 14, PW = Q4 ? 9 : 55;
+    uint32_t wr[NW], wc[NW];
 #pragma unroll
-        for (int k = 0; k < NP / 2; k++) v[k] = pp[NT * k];
-        if (h) v[NP / 2] = reinterpret_cast<const u32x4*>(A.side)[(size_t)sb * NX + min(tid, NX - 1)];
-    };
-    auto sstore = [&](int h, int buf, const u32x4 (&v)[NH]) {
+    for (int i = 0; i < NW; i++) {
+        const int c = min(lane + 64 * i, 16 * TL * PW - 1);
+        wr[i] = c / PW;
+        wc[i] = c - PW * wr[i];
+    }
+    uint8_t* const wl = smem + WL + wave * WB;
+    auto load_w = [&](int rb, int sb) {
+        const int r0 = min(rb * R + 16 * TL * wave, A.N - 1);         // uniform
+        const uint32_t last = (uint32_t)(A.N - 1 - r0);
+        const uint8_t* src = A.w + (size_t)r0 * rbytes + (size_t)sb * TI::BB;
+        const uint32_t dst = lds0 + (uint32_t)(WL + wave * WB);
+        if constexpr (Q4) {
+            if (A.walign) {                 // uniform
 #pragma unroll
-        for (int k = 0; k < NP / 2; k++) lds[buf * SU + tid + NT * (k + (NP / 2) * h)] = v[k];
-        if (h && tid < NX) lds[buf * SU + PU + tid] = v[NP / 2];
+                for (int i = 0; i < NW; i++)
+                    if (i < 4 || lane < 32)
+                        mf_glds16(dst + 1024 * i, min(wr[i], last) * (uint32_t)rbytes + 16 * wc[i], src);
+            } else {                        // addresses that such loads may not take: through registers
+#pragma unroll
+                for (int i = 0; i < NW; i++) {
+                    const uint4 v = ld16(to_global(src) + (min(wr[i], last) * (uint32_t)rbytes + 16 * wc[i]));
+                    if (i < 4 || lane < 32) *reinterpret_cast<uint4*>(wl + 1024 * i + 16 * lane) = v;
+                }
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // fewer loads than counted: wait here
+            }
+        } else {
+            // the dwords that hold the block (53; 54 if it starts 3 off), 55
+            // places a row: an odd count for the LDS banks; the places past
+            // the last hold it again
+            const uint32_t mis = (uint32_t)(uintptr_t)src & 3u;
+#pragma unroll
+            for (int i = 0; i < NW; i++) {
+                const uint32_t o = min(wr[i], last) * (uint32_t)rbytes + mis + (wc[i] > 52 ? 1u : 0u);
+                mf_glds4(dst + 256 * i, (o & ~3u) + 4 * min(wc[i], 52u), src - mis);
+            }
+        }
+    };
+    auto load_side = [&](int sb, int buf) {
+        const int pc = min(wave, (NX - 1) / 64);                      // a piece past the last: the last again
+        const int i = 64 * pc + lane;
+        if (i < NX)
+            mf_glds16(lds0 + (uint32_t)(SIDE + buf * NX * 16 + 1024 * pc), 16u * i,
+                      A.side + (size_t)sb * NX);
+    };
+    auto load_half = [&](int sb, int h, int slot) {
+        const uint4* src = A.planes + (size_t)sb * PU + 512 * h + 64 * wave;
+#pragma unroll
+        for (int g = 0; g < NSG; g++)
+            mf_glds16(lds0 + (uint32_t)(16 * (slot * HU + 512 * g + 64 * wave)), 16u * lane,
+                      src + MF_GROUP_U4 * g);
     };
     int rb = it0 / NSB, sb = it0 - rb * NSB;
-    typename MfRaw<TYPE>::T raw[TL];
-    {
-        u32x4 v0[NH], v1[NH];
-        sload(0, sb, v0);
-        sload(1, sb, v1);
-#pragma unroll
-        for (int t = 0; t < TL; t++) raw[t] = mf_load<TYPE>(wrow(rb, t) + (size_t)sb * TI::BB, kg);
-        sstore(0, 0, v0);
-        sstore(1, 0, v1);
-    }
-    __syncthreads();
+    load_w(rb, sb);
+    load_side(sb, 0);
+    load_half(sb, 0, 0);
+    load_half(sb, 1, 1);
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 acc[TL][NSG];
 #pragma unroll
     for (int t = 0; t < TL; t++)
 #pragma unroll
         for (int g = 0; g < NSG; g++) acc[t][g] = zero;
+    int slot = 0;                           // of this iteration's first half
     for (int it = it0; it < it1; it++) {
         const int buf = (it - it0) & 1;
         const bool more = it + 1 < it1;
         const int sbn = sb + 1 == NSB ? 0 : sb + 1, rbn = sb + 1 == NSB ? rb + 1 : rb;
         const int sbl = more ? sbn : sb, rbl = more ? rbn : rb;   // the last iteration reloads its own
+        const int slot1 = slot == 2 ? 0 : slot + 1, slot2 = slot1 == 2 ? 0 : slot1 + 1;
+        mf_wait_barrier<NSG>();             // all but the second half is in; slot2 and the other side are free
         typename MfRaw<TYPE>::T rc[TL];
         MfSb<TYPE> cs[TL];
 #pragma unroll
         for (int t = 0; t < TL; t++) {
-            rc[t] = raw[t];
-            cs[t] = mf_sb(rc[t], kg);
+            if constexpr (Q4) rc[t] = mf_read_q4k(wl, 16 * t + (lane & 15), kg);
+            else {
+                const int row = min(rb * R + 16 * wave + (lane & 15), A.N - 1);
+                const uint32_t at = (uint32_t)(uintptr_t)A.w + (uint32_t)row * (uint32_t)rbytes +
+                                    (uint32_t)sb * (uint32_t)TI::BB;
+                rc[t] = mf_read_q6k(wl, lane & 15, kg, 8u * (at & 3u));
+            }
         }
-        u32x4 sv[NH];
-        sload(0, sbl, sv);                  // the next stage's first half, then the next weights
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's weights are read: its LDS takes the next
+        load_w(rbl, sbl);
+        load_side(sbl, buf ^ 1);
+        load_half(sbl, 0, slot2);
 #pragma unroll
-        for (int t = 0; t < TL; t++) raw[t] = mf_load<TYPE>(wrow(rbl, t) + (size_t)sbl * TI::BB, kg);
+        for (int t = 0; t < TL; t++) cs[t] = mf_sb(rc[t], kg);
         f32x4 C[TL][NSG], D[TL][NSG];       // D: the Q6_K sl parts
 #pragma unroll
         for (int t = 0; t < TL; t++)
 #pragma unroll
             for (int g = 0; g < NSG; g++) C[t][g] = D[t][g] = zero;
-        const u32x4* sp = lds + buf * SU + lane;
         // step j + 1's plane reads and weight decode are issued while step
         // j's MFMAs run
         half8 x0[2][NSG], x1[2][NSG], wa[2][TL], wb[2][TL];
         auto fetch = [&](int j, int c) {
+            const u32x4* sp = lds + (j < 4 ? slot : slot1) * HU + (j & 3) * 128 + lane;
 #pragma unroll
             for (int g = 0; g < NSG; g++) {
-                x0[c][g] = __builtin_bit_cast(half8, sp[(g * 8 + j) * 128]);
-                x1[c][g] = __builtin_bit_cast(half8, sp[(g * 8 + j) * 128 + 64]);
+                x0[c][g] = __builtin_bit_cast(half8, sp[g * 512]);
+                x1[c][g] = __builtin_bit_cast(half8, sp[g * 512 + 64]);
             }
 #pragma unroll
             for (int t = 0; t < TL; t++) {
@@ -2969,6 +3033,10 @@ __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int c = j & 1;
+            if (j == 3) {                   // steps 0-3 are read: the second half in, the next one's to its place
+                mf_wait_barrier<NW + 1 + NSG>();
+                load_half(sbl, 1, slot);
+            }
             if (j < 7) fetch(j + 1, c ^ 1);
             // every accumulator once per pass, so dependent MFMAs are
             // TL * NSG instructions apart
@@ -2984,10 +3052,6 @@ __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
                             D[t][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa, wb[c][t], D[t][g], 0, 0, 0);
                     }
             }
-            if (j == 3) {                   // the first half is in: store it, fetch the second
-                sstore(0, buf ^ 1, sv);
-                sload(1, sbl, sv);
-            }
             // keeps the compiler from hoisting later steps' reads (registers)
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -2995,7 +3059,7 @@ __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
         // min term
 #pragma unroll
         for (int g = 0; g < NSG; g++) {
-            const u32x4* sd = lds + buf * SU + PU + MF_SIDE_U4 * g;
+            const u32x4* sd = lds + SIDE / 16 + buf * NX + MF_SIDE_U4 * g;
             const float a0 = reinterpret_cast<const float*>(sd)[lane];
             const float a1 = reinterpret_cast<const float*>(sd)[64 + lane];
             const u32x4 e4 = sd[32 + kg];         // E of streams 4 kg + v
@@ -3020,7 +3084,6 @@ __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
                 acc[t][g] = s;
             }
         }
-        sstore(1, buf ^ 1, sv);             // unused after the last iteration
         if (sb == NSB - 1 || !more) {       // the row block's sums: y, or a partial
             const long a0 = (long)rb * NSB;
             const bool own = A.whole || mf_owner(a0, A.T, A.G) == mf_owner(a0 + NSB - 1, A.T, A.G);
@@ -3046,8 +3109,9 @@ __global__ __launch_bounds__(64 * MF_NW) void kq_mf_kernel(MfArg A) {
         }
         rb = rbn;
         sb = sbn;
-        __syncthreads();
+        slot = slot2;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last reloads
 }
 
 // y of the row blocks that several workgroups share: their partial sums
@@ -3097,7 +3161,8 @@ int launch_mfma_t(const float* x, const void* w, float* y, int B, int N, int K, 
     a.side = s.side; a.y = y; a.part = part;
     a.B = B; a.N = N; a.K = K; a.NSG = NSG;
     a.nrb = p.nrb; a.G = p.G; a.whole = p.whole; a.T = p.T;
-    const size_t lds = (size_t)2 * mf_stage_u4(NSG) * 16;
+    a.walign = ((uintptr_t)w & 15) == 0;
+    const size_t lds = mf_lds<TYPE>(NSG);
     typedef void (*mf_fn)(MfArg);
     const mf_fn fn[4] = {&kq_mf_kernel<TYPE, 1>, &kq_mf_kernel<TYPE, 2>, &kq_mf_kernel<TYPE, 3>,
                          &kq_mf_kernel<TYPE, 4>};

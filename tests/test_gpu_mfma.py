@@ -153,6 +153,22 @@ def test_mfma_wide_dynamic_range(port, qtype):
     assert (err[live] / mag[live]).max() <= TOL
 
 
+@pytest.mark.parametrize("qtype,off", [(12, 2), (12, 4), (12, 8), (12, 16), (14, 1), (14, 2), (14, 3), (14, 6)])
+@pytest.mark.parametrize("B,N,Kd", [(16, 300, 512), (50, 5, 1280), (64, 257, 256)])
+def test_mfma_weight_addresses(qtype, off, B, N, Kd):
+    """Weights at any address (16-byte loads straight to LDS where they may be
+    used, registers elsewhere; Q6_K's dwords from any byte) give the same bits."""
+    w = torch.from_numpy(synth.tensor(qtype, N, Kd, 990 + off)).cuda()
+    xs = np.stack([synth.gaussian(synth.rng(970 + s), Kd) for s in range(B)])
+    buf = torch.empty(w.numel() + 64, dtype=torch.uint8, device="cuda")
+    assert buf.data_ptr() % 64 == 0
+    buf[off:off + w.numel()] = w
+    want = run(K.gemv_multix_mfma_dev, qtype, w, xs, B, N, Kd)
+    got = run(K.gemv_multix_mfma_dev, qtype, buf[off:], xs, B, N, Kd)
+    assert np.all(np.isfinite(want))
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_mfma_repeatable_and_other_types_refused():
     """Two launches give the same bits (the partial sums are added in a
     fixed order); types without a matrix-core path return -1."""
