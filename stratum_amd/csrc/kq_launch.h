@@ -76,6 +76,7 @@ int kqk_mx_set_max_lds(int bytes);
  * -1: not taken), and the launch (x_j = X + j x_stride, y_j = Y + j y_stride) */
 #define KQK_MV_PLAN 5
 long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan);
+int kqk_mv_slots(const int* plan, int M);
 int kqk_mv_set_max_lds(int bytes);
 int kqk_launch_mv(int type, const int* plan, long lds, const void* w, const float* X, long x_stride,
                   float* Y, long y_stride, int M, int N, int K, hipStream_t st);

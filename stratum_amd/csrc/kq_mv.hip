@@ -361,6 +361,13 @@ __host__ __device__ __forceinline__ int mv_cut(int S, int rem, int W) {
     return S * rem <= W ? S : S == 4 && 2 * rem <= W ? 2 : 1;
 }
 
+// Where a task of streams m0 .. m0 + n - 1 starts: one that would read past the
+// last x slot (S = 3: streams 6, 7 and 8 of 8) takes the last n slots, and does
+// not store the streams before m0.
+__host__ __device__ __forceinline__ int mv_x0(int m0, int n) {
+    return m0 < MV_ME - n ? m0 : MV_ME - n;
+}
+
 // A copy the optimiser takes for new values: the variants of a unit would
 // otherwise have their common decode hoisted above the branch, all at once.
 template <typename R> __device__ __forceinline__ R mv_opaque(const R& r) {
@@ -417,6 +424,7 @@ void kq_mv_kernel(MvArg A) {
     // odd workgroups fill their waves from the other end
     const int w0 = (blockIdx.x >> 3) & 1 ? W - 1 - wave : wave;
     MvTasks tk;
+    [[maybe_unused]] int own[MV_TW];               // the first stream to store (mv_x0)
     tk.kb = w0 < rem * cut ? 0 : 1;
     tk.ke = full + 1;
     tk.n0 = S / cut;
@@ -425,6 +433,10 @@ void kq_mv_kernel(MvArg A) {
         const int t = k ? rem + w0 + (k - 1) * W : w0 / cut;
         tk.grp[k] = t / nsg;
         tk.m0[k] = (t - tk.grp[k] * nsg) * S + (k ? 0 : (w0 % cut) * tk.n0);
+        if constexpr (MV_ME % S != 0) {
+            own[k] = tk.m0[k];
+            tk.m0[k] = mv_x0(own[k], k ? S : tk.n0);
+        }
     }
     const wptr gw = to_global(A.w);
     auto wrow = [&](int k) {
@@ -542,7 +554,8 @@ void kq_mv_kernel(MvArg A) {
             for (int s = 0; s < S; s++) {
                 const double v = phase_tree(part[k][s], GP);
                 const int m = tk.m0[k] + s, rr = RPT * tk.grp[k] + lr;
-                if (p == 0 && rr < rows && m < Mc && (k > 0 || s < tk.n0))
+                if (p == 0 && rr < rows && m < Mc && (k > 0 || s < tk.n0) &&
+                    (MV_ME % S == 0 || m >= own[k]))
                     A.Y[(size_t)(m0 + m) * A.y_stride + r0 + rr] = (float)v;
             }
         }
@@ -626,6 +639,23 @@ long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan
         }
     }
     return best_lds;
+}
+
+// x slots that the tasks of a plan's launch read (MV_ME are staged): every
+// group of S streams of its stream chunks, whole and in pieces
+int kqk_mv_slots(const int* plan, int M) {
+    const int S = plan[4];
+    int top = 0;
+    for (int c = 0; c < plan[1]; c++) {
+        const int Mc = c + 1 < plan[1] ? plan[0] : M - c * plan[0];
+        for (int m0 = 0; m0 < Mc; m0 += S)
+            for (int n = 1; n <= S; n++)
+                for (int i = 0; S % n == 0 && i < S; i += n) {
+                    const int t = (MV_ME % S ? mv_x0(m0 + i, n) : m0 + i) + n;
+                    if (t > top) top = t;
+                }
+    }
+    return top;
 }
 
 int kqk_mv_set_max_lds(int bytes) {

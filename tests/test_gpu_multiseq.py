@@ -31,6 +31,17 @@ def device():
                                     (3, 8448, 4), (65, 10496, 9), (1031, 768, 13),
                                     (2050, 2304, 17)])
 def test_multiseq_edges(qtype, N, Kd, B):
+    check(qtype, N, Kd, B)
+
+
+# groups of three with seven and eight streams staged: the last group starts
+# two streams before the last slot
+@pytest.mark.parametrize("qtype,N,Kd,B", [(14, 815, 16640, 16), (11, 815, 13568, 8)])
+def test_multiseq_last_group_of_three(qtype, N, Kd, B):
+    check(qtype, N, Kd, B)
+
+
+def check(qtype, N, Kd, B):
     w = synth.tensor(qtype, N, Kd, 4100 + qtype)
     xs = np.stack([synth.gaussian(synth.rng(4200 + s), Kd) for s in range(B)])
     xs[0, 5] = np.float32(1e-42)                 # subnormal
