@@ -601,6 +601,7 @@ long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan
     const double mem = xpc == 4 || type == T_Q6K ? 370 : 340;
     double best = 1e300;
     long best_lds = -1;
+    int best_wgs = 0;
     int nmc0 = (M + MV_ME - 1) / MV_ME;
     while (nmc0 < M && tiles + (M + nmc0 - 1) / nmc0 * xsum > lds_max) nmc0++;
     for (int nmc = nmc0; nmc <= M && nmc <= nmc0 + 1; nmc++) {
@@ -616,6 +617,11 @@ long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan
                 const long items = (long)((Q + ng - 1) / ng) * nmc, slots = (long)res * n_cu;
                 const long rounds = (items + slots - 1) / slots, last = items - (rounds - 1) * slots;
                 const int nt = ng * nsg, full = nt / W, rem = nt - full * W, cut = mv_cut(S, rem, W);
+                // one group of four streams of Q5_K, whose S = 4 form spills,
+                // unless every wave of two workgroups a CU has one: 17408 x 5120
+                // 48.1 us (44.4 as two groups of two), 11007 x 4096 30.6 (25.1);
+                // 32000 x 768, 500 items of 8 tasks, 16.2 (16.9)
+                if (type == T_Q5K && M == 4 && S == 4 && (rem || items <= n_cu)) continue;
                 // a turn of n waves on a SIMD takes max(2, n) of a wave's
                 // clocks at the full issue rate, which needs two waves
                 auto turn = [&](int wgs, int waves, int s) {
@@ -625,12 +631,23 @@ long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan
                 auto round_cost = [&](int wgs) {
                     const double t =
                         full * turn(wgs, W, S) + (rem ? turn(wgs, rem * cut, S / cut) : 0.0);
-                    return nstep * t + 12000.0;
+                    // a CU's only workgroup with half its waves idle waits out
+                    // its loads: 2560 x 9728 Q8_0 B = 3 in 6 waves of three
+                    // streams 21.6 us, in 15 of one 17.7 (the model: even)
+                    const bool few = H == 2 && !full && 2 * rem * cut <= W;
+                    return nstep * (few ? 1.3 * t : t) + 12000.0;
                 };
-                const double cost =
-                    (rounds - 1) * round_cost(res) + round_cost((int)((last + n_cu - 1) / n_cu));
-                if (cost < best) {
+                const int wgs = (int)((last + n_cu - 1) / n_cu);
+                const double cost = (rounds - 1) * round_cost(res) + round_cost(wgs);
+                // at one cost (the same pieces in a SIMD), fewer workgroups on a
+                // CU: each stages x for itself.  4096 x 4096 Q5_K B = 4 in 512
+                // items of one row group 22.9 us, in 256 of two 17.2.  Not where
+                // that leaves a turn of few waves: 11007 x 4096 Q2_K B = 5, 459
+                // items of 6 tasks 29.4, 230 of 12 on 8 waves 31.8
+                if (cost < best ||
+                    (cost == best && S == plan[4] && wgs < best_wgs && (!full || !rem))) {
                     best = cost;
+                    best_wgs = wgs;
                     best_lds = lds;
                     plan[0] = mc; plan[1] = nmc; plan[2] = ng; plan[3] = (Q + ng - 1) / ng;
                     plan[4] = S;

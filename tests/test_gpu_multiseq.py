@@ -35,8 +35,8 @@ def test_multiseq_edges(qtype, N, Kd, B):
 
 
 # groups of three with seven and eight streams staged: the last group starts
-# two streams before the last slot
-@pytest.mark.parametrize("qtype,N,Kd,B", [(14, 815, 16640, 16), (11, 815, 13568, 8)])
+# before its own streams, at the last three slots
+@pytest.mark.parametrize("qtype,N,Kd,B", [(14, 815, 16640, 16), (11, 815, 13568, 14), (12, 815, 9216, 16)])
 def test_multiseq_last_group_of_three(qtype, N, Kd, B):
     check(qtype, N, Kd, B)
 

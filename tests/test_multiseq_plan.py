@@ -18,8 +18,8 @@ def plan(qtype, N, Kd, B):
     return L.kqk_mv_plan(qtype, N, Kd, B, N_CU, LDS, p), p
 
 
-# the first two plan chunks of eight and of seven streams in groups of three
-@pytest.mark.parametrize("qtype,N,Kd,B", [(14, 815, 16640, 16), (11, 815, 13568, 8)])
+# chunks of eight and of seven streams in groups of three
+@pytest.mark.parametrize("qtype,N,Kd,B", [(14, 815, 16640, 16), (11, 815, 13568, 14), (12, 815, 9216, 16)])
 def test_slots_of_groups_of_three(qtype, N, Kd, B):
     lds, p = plan(qtype, N, Kd, B)
     assert lds > 0 and p[4] == 3 and p[0] >= 7
@@ -37,3 +37,23 @@ def test_slots_over_shapes():
         seen.add((p[0], p[4]))
         assert 1 <= K.lib().kqk_mv_slots(p, B) <= 8, (t, N, Kd, B, list(p))
     assert {(7, 3), (8, 3), (8, 4), (8, 2)} <= seen
+
+
+# the plans of calls that ran slower than one launch of the multi-x kernel: of
+# equal costs the one with fewer workgroups on a CU, no S = 4 for one group of
+# four streams of Q5_K, not half the waves of a CU's only workgroup idle
+@pytest.mark.parametrize("qtype,N,Kd,B,items", [(13, 4096, 4096, 4, 256), (8, 4096, 4096, 2, 256),
+                                                (11, 3000, 3072, 2, 188), (13, 17408, 5120, 4, None),
+                                                (13, 11007, 4096, 4, None), (8, 2560, 9728, 3, None)])
+def test_plans_of_few_streams(qtype, N, Kd, B, items):
+    lds, p = plan(qtype, N, Kd, B)
+    mc, nmc, ng, nblk, S = p
+    assert lds > 0 and nmc == 1
+    if items:
+        assert nblk == items
+    if qtype == 13:
+        assert S != 4
+    if Kd > 8192:                    # 16 waves, 2 rows a task
+        tasks = ng * -(-mc // S)
+        cut = S if S * tasks <= 16 else 1
+        assert tasks > 16 or 2 * tasks * cut > 16
