@@ -678,17 +678,25 @@ int kq_gemv_multix_dev(int type, const void* w, const float* xs, float* ys,
                 return -1;
         return 0;
     }
+    int s0 = 0;
     if (!(type & KQ_INT8_ACT)) {
-        int plan[KQK_MV_PLAN];
-        const long lds = mv_plan(type, N, K, B, plan);
-        if (lds > 0) {
-            const int e = kqk_launch_mv(type, plan, lds, w, xs, K, ys, N, B, N, K, pick(stream));
+        /* one launch, or, past a launch's size, equal parts that fit */
+        for (int nb = B; s0 < B; s0 += nb) {
+            int plan[KQK_MV_PLAN];
+            if (nb > B - s0) nb = B - s0;
+            long lds = mv_plan(type, N, K, nb, plan);
+            while (lds < 0 && nb > 8) {
+                nb = (nb / 2 + 7) & ~7;
+                lds = mv_plan(type, N, K, nb, plan);
+            }
+            if (lds < 0) break;
+            const int e = kqk_launch_mv(type, plan, lds, w, xs + (size_t)s0 * K, K,
+                                        ys + (size_t)s0 * N, N, nb, N, K, pick(stream));
             if (e) return kq_fail("multix launch: %s", hipGetErrorString((hipError_t)e));
-            return 0;
         }
     }
     const int grid = plan_grid();
-    for (int s0 = 0; s0 < B; ) {
+    while (s0 < B) {
         const int nb = B - s0 < 64 ? B - s0 : 64;
         int plan[KQK_MX_PLAN];
         static const int no_moe[4] = {0, 0, 0, 0};

@@ -335,6 +335,7 @@ KQ_MV_RAW(T_Q80, RawQ8, load_q80)
 // ------------------------------------------------------------- the kernel
 constexpr int MV_ME = 8;          // streams staged together
 constexpr int MV_TW = 2;          // tasks per wave, at most
+constexpr long MV_LANES = 1L << 32;   // of a launch (HIP refuses this many)
 
 struct MvArg {
     const uint8_t* w;
@@ -584,7 +585,9 @@ int mv_xpc(int type) {
 extern "C" {
 
 // Plan of an exact MULTISEQ launch: plan[] = streams per chunk, stream
-// chunks, row groups per item, items per stream chunk, S.  Returns the LDS bytes, or -1 when the kernel does not take it.
+// chunks, row groups per item, items per stream chunk, S.  Returns the LDS
+// bytes, or -1 when the kernel does not take it: x sums that leave no room for
+// the tiles, or more workgroups than a launch holds (fewer streams may fit).
 long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan) {
     if (mv_type(type) < 0 || N < 1 || M < 1 || K <= 0 || (K & 255)) return -1;
     const int NC = K >> 6, H = kq_phases(NC) == 32 ? 2 : 1;
@@ -615,6 +618,7 @@ long kqk_mv_plan(int type, int N, int K, int M, int n_cu, int lds_max, int* plan
             const int nsg = (mc + S - 1) / S;
             for (int ng = 1; ng * nsg < W * MV_TW; ng++) {
                 const long items = (long)((Q + ng - 1) / ng) * nmc, slots = (long)res * n_cu;
+                if ((items + 7) * 512 * H >= MV_LANES) continue;
                 const long rounds = (items + slots - 1) / slots, last = items - (rounds - 1) * slots;
                 const int nt = ng * nsg, full = nt / W, rem = nt - full * W, cut = mv_cut(S, rem, W);
                 // one group of four streams of Q5_K, whose S = 4 form spills,

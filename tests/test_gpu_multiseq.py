@@ -60,3 +60,23 @@ def check(qtype, N, Kd, B):
     got, one = got.cpu().numpy(), one.cpu().numpy()
     for j in range(B):
         assert same_values(got[j], one[j]), f"stream {j}"
+
+
+def test_multiseq_past_one_launch():
+    """More streams than the lanes of a launch hold go in parts.  Sixteen
+    different streams over and over: every one equals its single launch."""
+    N, Kd, B = 151936, 256, 32016
+    if torch.cuda.mem_get_info()[0] < 30 << 30:
+        pytest.skip("needs 20 GB")
+    rows = 64
+    w = torch.from_numpy(synth.tensor(12, rows, Kd, 4300)).cuda().repeat(N // rows)
+    x16 = torch.from_numpy(np.stack([synth.gaussian(synth.rng(4400 + s), Kd) for s in range(16)])).cuda()
+    dx, y = x16.repeat(B // 16, 1), torch.empty(B, N, device="cuda")
+    one = torch.empty(16, N, device="cuda")
+    print(f"multiseq Q4_K {N}x{Kd} B={B}", flush=True)
+    s = torch.cuda.current_stream().cuda_stream
+    K.gemv_multix_dev(12, w.data_ptr(), dx.data_ptr(), y.data_ptr(), B, N, Kd, stream=s)
+    for j in range(16):
+        K.gemv_dev(12, w.data_ptr(), x16[j].data_ptr(), one[j].data_ptr(), N, Kd, stream=s)
+    for j in range(0, B, 16):
+        assert torch.equal(y[j:j + 16], one), f"streams {j} ..."

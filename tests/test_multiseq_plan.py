@@ -57,3 +57,21 @@ def test_plans_of_few_streams(qtype, N, Kd, B, items):
         tasks = ng * -(-mc // S)
         cut = S if S * tasks <= 16 else 1
         assert tasks > 16 or 2 * tasks * cut > 16
+
+
+# very large batches: a plan's grid stays below the 2^32 lanes of a launch, and
+# where the whole batch does not fit, a half, a quarter, ... of it does
+@pytest.mark.parametrize("qtype,N,Kd,B", [(12, 151936, 8448, 8192), (12, 151936, 1024, 32768),
+                                          (14, 151936, 8448, 8192), (10, 32000, 17408, 131072),
+                                          (12, 8, 256, 1 << 28)])
+def test_plans_of_large_batches(qtype, N, Kd, B):
+    lanes = 1024 if Kd > 8192 else 512
+    nb = B
+    while True:
+        lds, p = plan(qtype, N, Kd, nb)
+        if lds > 0:
+            break
+        assert nb > 64
+        nb = (nb // 2 + 7) & ~7
+    assert (p[3] * p[1] + 7) // 8 * 8 * lanes < 1 << 32
+    assert p[0] * p[1] >= nb
