@@ -104,11 +104,12 @@ int kqk_noalloc_scratch(void** ptr, long* bytes);
 int kqk_launch_mfma(int type, const float* x, const void* w, float* y, int B, int N, int K,
                     void* planes, float* xs, float* part, int grid, hipStream_t st);
 /* int8 MULTISEQ on the matrix cores (kq_mi.hip; Q4_K / Q6_K | KQ_INT8_ACT,
- * B >= 2): workspace bytes or -1; the launch (prep + main kernel) with ws
- * 256-byte aligned.  kqk_mi8_parts: K-parts per row block (1, 2 or 4), by
+ * B >= 2): workspace bytes or -1; the launch (prep + main kernel) of up to
+ * kqk_mi_streams of the call's streams, with ws 256-byte aligned.  kqk_mi8_parts: K-parts per row block (1, 2 or 4), by
  * the row length only -- the grouping of the binary64 sums follows it */
 int kqk_mi8_parts(int K);
 long kqk_mi_workspace(int type, int B, int K);
+int kqk_mi_streams(int N, int K);
 int kqk_mi_set_max_lds(int bytes);
 int kqk_launch_mi(int type, const float* xs, long x_stride, const void* w, float* ys, long y_stride,
                   int B, int N, int K, void* ws, hipStream_t st);

@@ -650,12 +650,17 @@ static int mfma_reserve(kq_scr* sc, size_t need);
  * reference's multix_pack arithmetic. */
 static int mi8_multix(int type, const void* w, const float* xs, float* ys, int B, int N, int K,
                       hipStream_t st) {
-    const long need = kqk_mi_workspace(type, B, K);
+    const int most = kqk_mi_streams(N, K);      /* of one launch */
+    const long need = kqk_mi_workspace(type, B < most ? B : most, K);
     if (need < 0) return kq_fail("int8 multix: bad shape B=%d K=%d", B, K);
     kq_scr* sc = scr_of(st);
     if (!sc || mfma_reserve(sc, (size_t)need)) return -1;
-    const int e = kqk_launch_mi(type, xs, K, w, ys, N, B, N, K, sc->mf, st);
-    if (e) return kq_fail("int8 multix launch: %s", hipGetErrorString((hipError_t)e));
+    for (int s0 = 0, nb; s0 < B; s0 += nb) {
+        nb = B - s0 < most ? B - s0 : most;
+        const int e = kqk_launch_mi(type, xs + (size_t)s0 * K, K, w, ys + (size_t)s0 * N, N, nb, N, K,
+                                    sc->mf, st);
+        if (e) return kq_fail("int8 multix launch: %s", hipGetErrorString((hipError_t)e));
+    }
     return 0;
 }
 

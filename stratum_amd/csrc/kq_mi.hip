@@ -368,11 +368,20 @@ int kqk_mi_set_max_lds(int bytes) {
     return 0;
 }
 
+// Most streams of one launch, in whole sets: HIP refuses 2^32 lanes (2^24
+// workgroups of 256); 2^16 sets also bound the prep launch
+int kqk_mi_streams(int N, int K) {
+    const int rb = 4 / kqk_mi8_parts(K);
+    const long groups = ((N + 15L) / 16 + rb - 1) / rb, sets = ((1L << 24) - 8) / groups;
+    return (int)(16 * (sets < 1 ? 1 : sets > 1 << 16 ? 1 << 16 : sets));
+}
+
 int kqk_launch_mi(int type, const float* xs, long x_stride, const void* w, float* ys, long y_stride,
                   int B, int N, int K, void* ws, hipStream_t st) {
     const int ks = kqk_mi8_parts(K), nset = (B + 15) / 16;
-    if (kqk_mi_workspace(type, B, K) < 0 || N < 1 || B < 2 || (x_stride & 3) || x_stride < K ||
-        y_stride < N || ((uintptr_t)xs & 15) || ((uintptr_t)ws & 255) || ks > 4 || B > 65535 * 16)
+    if (kqk_mi_workspace(type, B, K) < 0 || N < 1 || B < 1 || (x_stride & 3) || x_stride < K ||
+        y_stride < N || ((uintptr_t)xs & 15) || ((uintptr_t)ws & 255) || ks > 4 ||
+        B > kqk_mi_streams(N, K))
         return (int)hipErrorInvalidValue;
     uint8_t* rec = static_cast<uint8_t*>(ws);
     if (type == T_Q4K_I8)
@@ -390,7 +399,7 @@ int kqk_launch_mi(int type, const float* xs, long x_stride, const void* w, float
     a.N = N; a.K = K; a.B = B; a.nset = nset;
     a.walign = ((uintptr_t)w & 15) == 0;
     const int rb = 4 / ks;
-    const long wgs = ((N + 15) / 16 + rb - 1) / rb * (long)nset;
+    const long wgs = ((N + 15L) / 16 + rb - 1) / rb * nset;
     hipLaunchKernelGGL(k_mi[type == T_Q6K_I8][ks == 4 ? 2 : ks - 1], dim3((unsigned)((wgs + 7) & ~7L)),
                        dim3(256), (size_t)mi_lds(type, ks), st, a);
     return (int)hipGetLastError();

@@ -45,3 +45,25 @@ def test_int8_multiseq_edges(port, qtype, N, Kd, B, off):
                       stream=torch.cuda.current_stream().cuda_stream)
     want = port.gemv_i8_multix(qtype, w, xs, N, Kd)
     assert same_values(got.cpu().numpy(), want)
+
+
+def test_int8_multiseq_past_one_launch(port):
+    """More streams than the lanes of a launch hold go in parts, the last of
+    one stream.  Sixteen different streams over and over: every one equals the
+    oracle's."""
+    N, Kd, rows = 151936, 12288, 64
+    B = K.lib().kqk_mi_streams(N, Kd) + 1
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 25 GB")
+    w = synth.tensor(12, rows, Kd, 5300)
+    x16 = np.stack([synth.gaussian(synth.rng(5400 + s), Kd) for s in range(16)])
+    want = torch.from_numpy(port.gemv_i8_multix(12, w, x16, rows, Kd)).cuda().repeat(1, N // rows)
+    dw = torch.from_numpy(w).cuda().repeat(N // rows)
+    dx = torch.from_numpy(x16).cuda().repeat(B // 16 + 1, 1)[:B].contiguous()
+    y = torch.empty(B, N, device="cuda")
+    print(f"int8 multiseq Q4_K {N}x{Kd} B={B}", flush=True)
+    K.gemv_multix_dev(12 | INT8_ACT, dw.data_ptr(), dx.data_ptr(), y.data_ptr(), B, N, Kd,
+                      stream=torch.cuda.current_stream().cuda_stream)
+    for j in range(0, B, 16):
+        n = min(16, B - j)
+        assert torch.equal(y[j:j + n], want[:n]), f"streams {j} ..."

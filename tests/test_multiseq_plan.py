@@ -1,5 +1,6 @@
-"""The exact MULTISEQ kernel's plans, on the host: every wave's tasks keep to
-the x slots that a workgroup stages (eight streams)."""
+"""The MULTISEQ kernels' plans, on the host: every wave's tasks keep to the x
+slots that a workgroup stages (eight streams), launches to the lanes that HIP
+takes."""
 import ctypes
 import random
 
@@ -75,3 +76,14 @@ def test_plans_of_large_batches(qtype, N, Kd, B):
         nb = (nb // 2 + 7) & ~7
     assert (p[3] * p[1] + 7) // 8 * 8 * lanes < 1 << 32
     assert p[0] * p[1] >= nb
+
+
+# the int8 kernel's most streams a launch: 256 lanes to every 64, 32 or 16 rows
+# (one, two or four K-parts) and 16 streams
+@pytest.mark.parametrize("N,Kd,rows", [(151936, 12288, 16), (151936, 4096, 32), (151936, 1024, 64),
+                                       (32000, 17408, 16), (1, 256, 64), (1 << 26, 256, 64)])
+def test_int8_streams_of_a_launch(N, Kd, rows):
+    most = K.lib().kqk_mi_streams(N, Kd)
+    assert most >= 16 and most % 16 == 0
+    wgs = -(-N // rows) * (most // 16)
+    assert (wgs + 7) // 8 * 8 * 256 < 1 << 32
