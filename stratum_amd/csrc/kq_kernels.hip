@@ -2874,11 +2874,11 @@ template <int TYPE> constexpr size_t mf_lds(int nsg) {
 // dst and src uniform
 __device__ __forceinline__ void mf_glds16(uint32_t dst, uint32_t off, const void* src) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(src) : "memory");
+                 :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(src) : "memory", "m0");
 }
 __device__ __forceinline__ void mf_glds4(uint32_t dst, uint32_t off, const void* src) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-                 :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(src) : "memory");
+                 :: "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(src) : "memory", "m0");
 }
 // at most N loads of this wave outstanding, its LDS reads done, then a barrier
 // that leaves those loads in flight

@@ -170,7 +170,7 @@ void kq_mi_kernel(MiArg A) {
     const uint8_t* w0 = A.w + (size_t)min(rb * 16, N - 1) * ((size_t)nb * BB);   // uniform
     auto glds = [&](uint32_t dst, uint32_t off, const uint8_t* src) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :: "s"(dst), "v"(off), "s"(src) : "memory");
+                     :: "s"(dst), "v"(off), "s"(src) : "memory", "m0");
     };
     auto stage = [&](int t, int buf) {
 #pragma unroll
@@ -202,7 +202,7 @@ void kq_mi_kernel(MiArg A) {
             for (int i = 0; i < NW; i++)
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                              :: "s"(dst + 256u * i), "v"(((wo[i] + mis) & ~3u) + wd[Q4 ? 0 : i]), "s"(al)
-                             : "memory");
+                             : "memory", "m0");
         }
     };
 

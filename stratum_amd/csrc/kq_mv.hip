@@ -470,7 +470,7 @@ void kq_mv_kernel(MvArg A) {
                         lds0 + (uint32_t)((ti & 1) * MV_ME + j) * Sh::XM + 1024u * cg;
                     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\t"
                                  "global_load_lds_dwordx4 %1, %2"
-                                 :: "s"(dst), "v"(voff), "s"(src) : "memory");
+                                 :: "s"(dst), "v"(voff), "s"(src) : "memory", "m0");
                 }
             }
         }
