@@ -635,3 +635,27 @@ def test_moe_int8_per_stream_types(port, qtype, H, F, N_g):
     dn = run_moe(qi, [down], sel, act, 1, B, k, n_exp, H, F)
     check_i8_tickets(port, qtype, down, sel, act, 1, dn[0], H, F, n_exp)
     assert np.isnan(dn[0][hole]).all()
+
+
+@pytest.mark.parametrize("qtype,H", [(12, 512), (14, 512), (10, 512), (13, 512), (11, 512), (8, 512), (42, 512),
+                                     (12, 40960), (14, 40960), (10, 40960), (13, 40960)])
+def test_moe_batch_out_of_window(port, qtype, H):
+    """One token with values outside the scaled window among runs of several
+    members (x staged whole, and, past a workgroup's LDS, in tiles): its runs
+    take the convert path.  Against each member's single launch bit for bit,
+    or, for rows too long for that launch, the oracle within the bound."""
+    E, F, B, k = 4, 96, 8, 2
+    w = experts(qtype, E, F, H, 51)
+    r = np.random.default_rng(52)
+    sel = np.stack([r.permutation(E)[:k] for _ in range(B)]).astype(np.int32)
+    xs = np.stack([synth.gaussian(r, H) for _ in range(B)])
+    xs[3, 17], xs[3, H - 5] = np.float32(2.0 ** 60), np.float32(2.0 ** -60)
+    print(f"moe window {K.TYPE_NAMES[qtype]} H={H}", flush=True)
+    got = run_moe(qtype, [w], sel, xs.reshape(-1), k, B, k, E, F, H)
+    if H == 512:
+        check_members(port, qtype, [w], sel, xs.reshape(-1), k, got, F, H)
+        return
+    sl = F * K.lib().kq_row_bytes(qtype, H)
+    for m, e in enumerate(sel.reshape(-1)):
+        want = port.gemv(qtype, w[e * sl:(e + 1) * sl], xs[m // k], F, H)
+        assert O.rel_err(got[0][m], want).max() <= 1e-5, (m, e)

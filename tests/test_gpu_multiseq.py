@@ -3,11 +3,15 @@ of 8 (at most 128 chunks) and 2 rows, tiles of 16 and 32 chunks, streams in
 groups of 2-4 and chunks of 8, one and many workgroups, special x values.
 Every stream equals its own single-stream launch bit for bit (the contract:
 tolerance none)."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import stratum_amd as K
 from conftest import same_values
+from mv_cases import ROWS, SHAPES, plans
+from oracle import oracle as O
 from stratum_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +43,68 @@ def test_multiseq_edges(qtype, N, Kd, B):
 @pytest.mark.parametrize("qtype,N,Kd,B", [(14, 815, 16640, 16), (11, 815, 13568, 14), (12, 815, 9216, 16)])
 def test_multiseq_last_group_of_three(qtype, N, Kd, B):
     check(qtype, N, Kd, B)
+
+
+# the layer shapes whose plans are the forms S = 3 and 4 of long rows, and S = 4
+# of Q2_K and type 42
+@pytest.mark.parametrize("qtype,N,Kd,B", [(12, 5120, 17408, 3), (12, 5120, 17408, 6)] +
+                         [(t, n, k, b) for t in (10, 42) for n, k in ((17408, 5120), (5120, 17408))
+                          for b in (8, 16)])
+def test_multiseq_layer_shapes(qtype, N, Kd, B):
+    check(qtype, N, Kd, B)
+
+
+@pytest.mark.parametrize("H", [1, 2])
+@pytest.mark.parametrize("qtype", [12, 14, 13, 11, 8, 10, 42])
+def test_multiseq_every_form(qtype, H):
+    """Every form of the kernel, launched with its plan (mv_cases): whole
+    items and a last one of two row groups and a row."""
+    L, Kd, (W, rpt) = K.lib(), ROWS[H], SHAPES[H]
+    L.kqk_mv_plan.restype = ctypes.c_long
+    L.kqk_launch_mv.argtypes = [ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.c_long, ctypes.c_void_p,
+                                ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p, ctypes.c_long, ctypes.c_int,
+                                ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    most = max(ng for h, _, ng, _, _ in plans() if h == H) * rpt + 2 * rpt + 1
+    B = max(M for _, _, _, _, M in plans())
+    w = torch.from_numpy(synth.tensor(qtype, most, Kd, 4500 + qtype)).cuda()
+    x = torch.from_numpy(np.stack([synth.gaussian(synth.rng(4600 + j), Kd) for j in range(B)])).cuda()
+    one = torch.empty(B, most, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    for j in range(B):
+        K.gemv_dev(qtype, w.data_ptr(), x[j].data_ptr(), one[j].data_ptr(), most, Kd, stream=s)
+    xpc = {12: 32, 13: 32, 10: 16, 42: 16}.get(qtype)              # x values of a sum
+    for h, S, ng, mc, M in plans():
+        if h != H:
+            continue
+        N = ng * rpt + min(ng, 2) * rpt + 1
+        groups = -(-N // rpt)
+        p = (ctypes.c_int * 5)(mc, -(-M // mc), ng, -(-groups // ng), S)
+        lds = 131072 * H // 2 + (mc * Kd // xpc * 4 if xpc else 0)   # x tiles, x sums
+        print(f"multiseq {K.TYPE_NAMES[qtype]} {N}x{Kd} M={M} plan={list(p)}", flush=True)
+        assert L.kqk_mv_slots(p, M) <= 8
+        got = torch.full((M, N), 7.0, device="cuda")
+        assert L.kqk_launch_mv(qtype, p, lds, w.data_ptr(), x.data_ptr(), Kd, got.data_ptr(), N, M, N, Kd, s) == 0
+        assert torch.equal(got, one[:M, :N]), (N, M, list(p))
+
+
+# rows too long for the single-stream launch: up to the x sums that leave room
+# for the tiles, and past them (Q4_K / Q5_K 262144, Q2_K / type 42 131072: the
+# multi-x kernel); a stream outside its scaled window.  Bound of the parity
+# tests.
+@pytest.mark.parametrize("qtype,Kd", [(12, 65536), (14, 131072), (12, 262400), (13, 262400), (10, 131328),
+                                      (42, 131328)])
+def test_multiseq_very_long_rows(port, qtype, Kd):
+    N, B = 5, 3
+    w = synth.tensor(qtype, N, Kd, 4700 + qtype)
+    xs = np.stack([synth.gaussian(synth.rng(4800 + s), Kd) for s in range(B)])
+    xs[1, 4097] = np.float32(2.0 ** -60)
+    print(f"multiseq {K.TYPE_NAMES[qtype]} {N}x{Kd} B={B}", flush=True)
+    dw, dx = torch.from_numpy(w).cuda(), torch.from_numpy(xs).cuda()
+    got = torch.full((B, N), 7.0, device="cuda")
+    K.gemv_multix_dev(qtype, dw.data_ptr(), dx.data_ptr(), got.data_ptr(), B, N, Kd,
+                      stream=torch.cuda.current_stream().cuda_stream)
+    for j in range(B):
+        assert O.rel_err(got[j].cpu().numpy(), port.gemv(qtype, w, xs[j], N, Kd)).max() <= 1e-5, f"stream {j}"
 
 
 def check(qtype, N, Kd, B):

@@ -531,8 +531,10 @@ def test_multix_bit_identical_to_single_stream(port, qtype, B, N, Kd):
 
 @pytest.mark.parametrize("qtype", [12, 10, 14, 13, 11, 8])
 def test_multix_window_fallback(port, qtype):
-    """One stream with a value outside the scaled window sends the launch to
-    the exact path; every stream still equals its single-stream result."""
+    """One stream with a value outside the single-stream kernel's scaled
+    window, which sends its own launch to the convert path: the streams of one
+    launch, which has no window, still equal their single-stream results.
+    (The multi-x kernel's window: test_moe_batch_out_of_window.)"""
     N, Kd, B = 80, 1024, 4
     w = synth.tensor(qtype, N, Kd, 830 + qtype)
     xs = np.stack([synth.gaussian(synth.rng(840 + s), Kd) for s in range(B)])
@@ -545,8 +547,8 @@ def test_multix_window_fallback(port, qtype):
 
 @pytest.mark.parametrize("qtype", [12, 10, 14, 42, 13, 11, 8])
 def test_multix_tiled_window_fallback(port, qtype):
-    """x too long to stage whole (tiles of a few chunks), with one stream
-    outside the scaled window: the tiled exact path, still bit-identical."""
+    """Many x tiles, with one stream outside the single-stream kernel's scaled
+    window: still bit-identical."""
     N, Kd, B = 200, 5120, 8
     w = synth.tensor(qtype, N, Kd, 870 + qtype)
     xs = np.stack([synth.gaussian(synth.rng(880 + s), Kd) for s in range(B)])
@@ -560,8 +562,8 @@ def test_multix_tiled_window_fallback(port, qtype):
 @pytest.mark.parametrize("qtype,B", [(12, 17), (12, 40), (12, 64), (12, 70), (13, 40), (11, 64),
                                      (8, 70)])
 def test_multix_member_chunks(port, qtype, B):
-    """More than 16 streams: members staged 16 at a time within one weight
-    pass (and more than 64 in two launches)."""
+    """More streams than are staged together (chunks of at most 8): several
+    items a row block."""
     N, Kd = 100, 1024
     w = synth.tensor(qtype, N, Kd, 890 + B)
     xs = np.stack([synth.gaussian(synth.rng(900 + s), Kd) for s in range(B)])

@@ -245,8 +245,9 @@ def test_moe_gather_other_types(port, qtype, B):
 @pytest.mark.parametrize("qtype", DENSE)
 @pytest.mark.parametrize("N,Kd", [(1, 256), (128, 768), (128, 2048), (1000, 4096), (37, 20480)])
 def test_dense_gemv(port, qtype, N, Kd):
-    """F16 / F32 rows, including K % 512 == 256 (an F16 step half full) and
-    K beyond what the kernel stages in LDS (x read from memory)."""
+    """F16 / F32 rows in launches of few rows, including K % 512 == 256 (an
+    F16 step half full) and many blocks of loads a row.  (Many rows, x in LDS
+    and past it: test_gpu_dense_rows.)"""
     w = synth.tensor(qtype, N, Kd, 800 + N)
     x = synth.gaussian(synth.rng(801 + Kd), Kd)
     print(f"dense type={qtype} N={N} K={Kd}", flush=True)

@@ -7,6 +7,7 @@ import random
 import pytest
 
 import stratum_amd as K
+from mv_cases import form, plans
 
 TYPES = (12, 14, 13, 11, 8, 10, 42)
 N_CU, LDS = 256, 163840          # the MI355X
@@ -87,3 +88,17 @@ def test_int8_streams_of_a_launch(N, Kd, rows):
     assert most >= 16 and most % 16 == 0
     wgs = -(-N // rows) * (most // 16)
     assert (wgs + 7) // 8 * 8 * 256 < 1 << 32
+
+
+def test_gpu_plans_cover_every_form():
+    """mv_cases' plans, which the GPU tests launch: every S at every row
+    length with no full turn and with one, its left-over tasks in every number
+    of pieces."""
+    seen = {(H, S) + form(H, S, ng, mc)[::2] for H, S, ng, mc, _ in plans()}
+    for H in (1, 2):
+        for S in (2, 3, 4):
+            cuts = {2: (1, 2), 3: (1, 3), 4: (1, 2, 4)}[S]
+            want = {(full, cut) for full in (0, 1) for cut in cuts} | {(1, 0)}
+            assert want <= {s[2:] for s in seen if s[:2] == (H, S)}, (H, S)
+    for H, S, ng, mc, M in plans():
+        assert ng * -(-mc // S) < 2 * {1: 8, 2: 16}[H] and mc <= 8 and mc <= M
