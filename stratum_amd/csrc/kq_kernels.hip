@@ -1761,8 +1761,10 @@ __global__ __launch_bounds__(1024) void kq_segs_kernel(SegsArg A) {
 
 // ------------------------------------------------------------- multi-x
 // y_j = W_g . x_j for the members j of each group g, with one pass over the
-// group's weight rows: STRATUM_MULTISEQ (one group, B members) and the MoE
-// gather (one group per selected expert, its routed tokens as members).
+// group's weight rows: the MoE gather (one group per selected expert, its
+// routed tokens as members), and STRATUM_MULTISEQ (one group, B members) in
+// the int8 mode of Q5_K, Q3_K and Q8_0; exact MULTISEQ is kq_mv.hip's, but for
+// rows whose x sums leave no room there (K past 262144, Q2_K / type 42 131072).
 // Each member's result is bit-identical to the single-stream kernel's for
 // the same row and x: the same chunk terms (same arithmetic, same x scaling
 // rule) and the same reduction (GP = kq_phases(K/64) partial sums over
@@ -3904,11 +3906,16 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
-// A few rows (a MoE router: at most DENSE_FEW_WAVES waves per CU): the launch
-// is one memory round trip, so a wave asks for BLK weight and x pieces of its
-// row at once, straight to registers, with no staging and no barrier.  The
-// sum runs in kq_dense_kernel's order.  128 x 2048 F32 (1 MB), B = 1, in a
-// MoE step: 7.2 us with x staged in LDS and the loads one at a time -> 3.9.
+// A few rows (a MoE router: at most DENSE_FEW_WAVES waves per CU, of any
+// length): such a launch is memory latency, so a wave asks for BLK weight and x
+// pieces of its row at once (2048 values), straight to registers, with no
+// staging and no barrier; longer rows take a round trip for each.  The sum
+// runs in kq_dense_kernel's order.  Against that kernel (x staged in LDS, or
+// past 16384 values read a piece at a time), F32 rows past the cache, us, B = 1:
+// 128 x 2048 5.3 -> 3.7, 256 x 8192 16.8 -> 7.2, 2048 x 2048 7.6 -> 5.1,
+// 2048 x 8192 23.1 -> 13.5, 2048 x 20480 50 -> 31; 256 x 8192 at B = 8, each
+// stream reading the weights again, 16.4 -> 7.7.  F16 2048 x 8192 15.3 -> 9.8.
+// Faster at all of 350 sizes of 8 to 2048 rows (times streams), K 512 to 20480.
 constexpr int DENSE_FEW_WAVES = 8;
 template <int TYPE>
 __global__ __launch_bounds__(256) void kq_dense_few_kernel(DenseArg a) {
@@ -4894,8 +4901,8 @@ int kqk_launch_dense(int type, const void* w, const float* x, const float* add, 
         return (int)hipGetLastError();
     }
     // DENSE_SB streams per wave share its weight loads, unless that leaves
-    // fewer than 8 waves per CU (a 128-row MoE router at B = 16: 256 waves
-    // of long serial chains); then one stream per wave
+    // fewer than 8 waves per CU (512 rows at B = 8: 512 waves of long serial
+    // chains); then one stream per wave
     const long w8 = (long)N * ((B + DENSE_SB - 1) / DENSE_SB);
     const int sb = B == 1 || w8 < 8L * 256 ? 1 : DENSE_SB;
     const bool lds = (long)sb * K <= DENSE_XLDS_MAX;

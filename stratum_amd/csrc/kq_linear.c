@@ -665,9 +665,10 @@ static int mi8_multix(int type, const void* w, const float* xs, float* ys, int B
 }
 
 /* B streams with one pass over the weights: exact block types in kq_mv.hip
- * (rows whose x sums leave no room for its tiles, and the int8 mode of Q5_K,
- * Q3_K and Q8_0, in the multi-x kernel); each stream's y equals its single-stream result bit
- * for bit, except in the int8 mode of Q4_K / Q6_K (mi8_multix). */
+ * (rows whose x sums leave no room for its tiles, K past 262144 or, Q2_K and
+ * type 42, 131072, and the int8 mode of Q5_K, Q3_K and Q8_0 in the multi-x
+ * kernel); each stream's y equals its single-stream result bit for bit,
+ * except in the int8 mode of Q4_K / Q6_K (mi8_multix). */
 int kq_gemv_multix_dev(int type, const void* w, const float* xs, float* ys,
                        int B, int N, int K, kq_stream stream) {
     if (B < 1) return kq_fail("kq_gemv_multix_dev: B=%d", B);

@@ -17,11 +17,14 @@
 // bytes of two sub-blocks are one 16-byte read.  (Q6_K's groups are half of
 // the 32 positions: the other half of the weights is zeroed, twice.)
 //
-// What bounds it: the weight stream (17408 x 5120 Q4_K: 50 MB, 10 us) and
-// 22 clk of VALU per (row, stream, sub-block), 6.4 us at 16 streams, and the
-// caches' accesses: a row to a lane, as the MFMA wants its operand, every
-// lane of a load is an access of its own (11 M a call at 16 streams, which
-// with loads a super-block ahead held it at 26 to 30 us).  So all loads go to
+// What bounds it.  At 64 streams VALU issue: 17408 x 5120 Q4_K 24.6 K
+// instructions a SIMD, 98 K clk of 58 us.  At 16 and fewer neither the weight
+// stream (50 MB, 10 us) nor VALU (6.1 K instructions a SIMD, 10 to 12 us of
+// 22.4): with two waves a SIMD, a wave waits in 37 % of its life for a step's
+// loads, which are asked for one super-block ahead and all awaited at the
+// step's barrier.  With the weights a row to a lane, as the MFMA wants its
+// operand, every lane of a load is a cache access of its own (11 M a call at
+// 16 streams, which held it at 26 to 30 us).  So all loads go to
 // LDS without registers (global_load_lds) in address order, neighbouring lanes
 // reading neighbouring bytes: one record per super-block and 16 streams,
 // shared by the workgroup's row blocks, and each wave's 16 weight blocks, a

@@ -18,14 +18,28 @@
 // against 7.5 for the byte-select form.  x needs no scaling window here: a
 // quant is converted, not read as a denormal.
 // The x tiles go from L2 to LDS without registers (global_load_lds), which
-// with S = 4 leaves 128 VGPRs, four waves per SIMD.
+// with S = 4 leaves 128 VGPRs, four waves per SIMD.  The S = 4 forms of Q6_K
+// and Q5_K do not quite fit them: 5 to 8 VGPRs spill, 24 to 36 bytes a lane
+// (with S = 3 nothing does, and 5120 x 17408 B = 64 takes 620 us instead of
+// 485).
 //
 // Measured against the multi-x kernel (kq_mx_kernel, byte-select products, x
-// staged through registers), weights past the cache, us: Q4_K 17408x5120 at
-// B = 2 / 4 / 8 / 16 / 64 30 / 41 / 80 / 150 / 573 -> 26 / 35 / 52 / 95 /
-// 340; Q6_K 5120x17408 at B = 2 / 8 / 13 / 64 57 / 132 / 247 / 1000 -> 38 /
-// 76 / 143 / 490; Q5_K 11007x4096 at B = 6 38 -> 32.  B = 8 on the gate is
-// 88 K clk of issue; the rest is uneven turns (17 tasks a CU) and the start.
+// staged through registers), weights past the cache, us at B = 2 / 4 / 8 / 16
+// / 64:
+//   17408 x 5120  Q4_K 32 / 41 / 80 / 151 / 572 -> 28 / 35 / 51 / 94 / 337
+//                 Q6_K 64 / 69 / 91 / 171 / 651 -> 39 / 50 / 70 / 113 / 418
+//                 Q5_K 32 / 47 / 88 / 171 / 664 -> 30 / 45 / 61 / 115 / 409
+//                 Q3_K 41 / 51 / 98 / 190 / 745 -> 34 / 45 / 65 / 110 / 380
+//                 Q8_0 33 / 40 / 77 / 145 / 553 -> 30 / 38 / 57 / 97 / 354
+//                 Q2_K 26.7 / 40 / 70 / 133 / 509 -> 27.2 / 36 / 52 / 95 / 341
+//                 type 42 31 / 40 / 75 / 141 / 535 -> 28 / 37 / 53 / 97 / 347
+//   5120 x 17408  Q4_K 30 / 59 / 108 / 205 / 788 -> 26 / 43 / 70 / 135 / 460
+//                 Q6_K 57 / 70 / 132 / 256 / 997 -> 38 / 52 / 73 / 141 / 485
+//                 Q2_K 31 / 46 / 85 / 163 / 634 -> 25 / 41 / 60 / 116 / 477
+// Over 16 shapes, 13 B and the seven types 1.4 to 1.9 times (geometric means by
+// type); slower in two of the 1456: Q8_0 17408 x 5120 B = 5 (46.8 -> 49.2) and
+// Q2_K 17408 x 5120 B = 2.  At B = 8 on the gate the SIMDs issue 32 K VALU
+// instructions each, about all of the kernel's clocks.
 // The same kernel with its products on the matrix cores (K = 1 MFMAs, C = 0,
 // which round like the multiply) took 59 and 104 us at B = 8 and 16.
 #include <hip/hip_runtime.h>
